@@ -14,9 +14,17 @@
 #include "../../include/culbm.h"
 #include "blocking.hpp"
 #include "lbm_kernels.hip"
+#include "fused.hip"
 #include "adjoint.hip"
 
 using namespace culbm;
+
+// Launch shape of k_fused2: tile, tile columns and rows, z planes per workgroup
+// and z chunks; `pays`: two steps in one launch beat two plain steps.
+struct FusedPlan {
+  int32_t tx = 0, ty = 0, tiles_x = 0, tiles_y = 0, zchunk = 0, nchunk = 0;
+  bool pays = false;
+};
 
 struct culbm_ctx {
   culbm_config cfg{};
@@ -44,9 +52,7 @@ struct culbm_ctx {
   float scale = 1.0f, inv_scale = 1.0f;
   double state_bound = 0.0;  // feq_bound over the cells of the last culbm_set_state
   int32_t wave_depth = 0;
-  // launch shape of k_fused2: tile columns and rows, z planes per workgroup and
-  // z chunks (the mixed policy; the adjoint's forward sweeps on every context)
-  int32_t tiles_x = 0, tiles_y = 0, fzchunk = 0, nchunk = 0;
+  FusedPlan fused;  // launch shape of k_fused2 (pull steps in pairs; the adjoint's forward sweeps)
   // static policy: one instantiated graph per starting state of a full pass
   // (pull: index of the current buffer; in-place: parity of the next step)
   hipGraphExec_t pass_graph[2] = {nullptr, nullptr};
@@ -524,41 +530,65 @@ int static_pass(culbm_ctx* ctx, int32_t T) {
   return CULBM_OK;
 }
 
-// Mixed blocking: two steps per launch with the intermediate in LDS, and one
-// plain step for an odd remainder.
+// k_fused2 computes on the populations in units of the storage scale, which
+// gives the bits of a plain step as long as neither side leaves the normal
+// range: FP16 holds multiples of 2^-24 below 2^16, so for scales 1 to 2^20
+// (every derived one) squares and cancelled sums of them stay above 2^-126;
+// BF16 reaches down to FP32's subnormals and has to be unscaled.  Any other
+// explicit scale runs plain steps.
+bool fused_scale_ok(const culbm_ctx* ctx) {
+  if (ctx->cfg.storage == CULBM_STORAGE_FP16) return ctx->scale >= 1.0f && ctx->scale <= 1048576.0f;
+  return ctx->scale == 1.0f;
+}
+
+// Two steps of the pull layout in one launch: a.src -> a.dst, producing the
+// states a.state and a.state + 1.
 template <class S>
-int fused_pass(culbm_ctx* ctx, int32_t T) {
+void launch_fused(const culbm_ctx* ctx, const StepArgs& a) {
+  const FusedPlan& p = ctx->fused;
   FusedArgs fa{};
-  fa.a = base_args(ctx);
-  fa.tiles_x = ctx->tiles_x;
-  fa.tiles_y = ctx->tiles_y;
-  fa.zchunk = ctx->fzchunk;
-  fa.nchunk = ctx->nchunk;
-  const uint32_t nblk = uint32_t(ctx->tiles_x) * ctx->tiles_y * ctx->nchunk;
-  for (int32_t s = 0; s + 1 < T; s += 2) {
-    fa.a.src = ctx->buf[ctx->cur];
-    fa.a.dst = ctx->buf[ctx->cur ^ 1];
-    fa.a.state = uint32_t(ctx->step) + 1u;  // the launch produces states state and state + 1
-    if (int rc = prof_begin(ctx)) return rc;
-    bool sr = false;
-    if constexpr (S::kBytes == 2) sr = ctx->sr;
-    if (sr)
-      hipLaunchKernelGGL((k_fused2<S, true>), dim3(nblk), dim3(FusedShape<S::kBytes>::BLOCK), 0, ctx->stream, fa);
-    else
-      hipLaunchKernelGGL((k_fused2<S, false>), dim3(nblk), dim3(FusedShape<S::kBytes>::BLOCK), 0, ctx->stream, fa);
-    HIPCHK(ctx, hipGetLastError());
-    if (int rc = prof_end(ctx)) return rc;
-    ctx->cur ^= 1;
-    ctx->step += 2;
+  fa.a = a;
+  fa.tx = p.tx;
+  fa.ty = p.ty;
+  fa.tiles_x = p.tiles_x;
+  fa.tiles_y = p.tiles_y;
+  fa.zchunk = p.zchunk;
+  fa.nchunk = p.nchunk;
+  const dim3 grid(uint32_t(p.tiles_x) * uint32_t(p.tiles_y) * uint32_t(p.nchunk));
+  const dim3 block(uint32_t(round_up(int64_t(p.tx + 2) * (p.ty + 2), 64)));
+  if constexpr (S::kBytes == 2) {
+    if (ctx->sr) {
+      hipLaunchKernelGGL((k_fused2<S, true>), grid, block, 0, ctx->stream, fa);
+      return;
+    }
   }
-  if (T & 1) {
-    StepArgs a = base_args(ctx);
+  hipLaunchKernelGGL((k_fused2<S, false>), grid, block, 0, ctx->stream, fa);
+}
+
+bool fused_pairs(const culbm_ctx* ctx);
+
+// Pull steps over the whole domain: in pairs where `pairs`, the odd one (and the
+// one a pending dump rides on) alone.
+template <class S>
+int pull_pass(culbm_ctx* ctx, int32_t T, bool pairs) {
+  StepArgs a = base_args(ctx);
+  while (T > 0) {
+    const bool pair = pairs && T > 1 && !ctx->dump_pending;
     a.src = ctx->buf[ctx->cur];
     a.dst = ctx->buf[ctx->cur ^ 1];
     a.state = uint32_t(ctx->step) + 1u;
-    if (int rc = launch_step<S>(ctx, a, 0, ctx->cfg.nz, 0)) return rc;
+    if (pair) {
+      if (int rc = prof_begin(ctx)) return rc;
+      launch_fused<S>(ctx, a);
+      HIPCHK(ctx, hipGetLastError());
+      if (int rc = prof_end(ctx)) return rc;
+    } else {
+      if (int rc = launch_step<S>(ctx, a, 0, ctx->cfg.nz, 0, ctx->dump_pending)) return rc;
+      ctx->dump_pending = false;
+    }
     ctx->cur ^= 1;
-    ctx->step += 1;
+    ctx->step += pair ? 2 : 1;
+    T -= pair ? 2 : 1;
   }
   return CULBM_OK;
 }
@@ -574,25 +604,21 @@ int do_steps(culbm_ctx* ctx, int32_t nsteps) {
     if (int rc = dump_impl<S>(ctx)) return rc;
     ctx->dump_pending = false;
   }
+  if (!ctx->inplace && (!blocked(c) || c.opt_policy == CULBM_OPT_MIXED || fused_pairs(ctx))) {
+    // the pairs run across the passes of innerLoop steps (the bits do not
+    // depend on the grouping)
+    return pull_pass<S>(ctx, nsteps, fused_pairs(ctx));
+  }
   if (!blocked(c)) {
     StepArgs a = base_args(ctx);
     for (int32_t s = 0; s < nsteps; ++s) {
-      if (!ctx->inplace) {
-        a.src = ctx->buf[ctx->cur];
-        a.dst = ctx->buf[ctx->cur ^ 1];
-      }
       a.state = uint32_t(ctx->step) + 1u;
       const int rc = launch_step<S>(ctx, a, 0, c.nz, ctx->parity, ctx->dump_pending);
       if (rc) return rc;
       ctx->dump_pending = false;
-      ctx->cur ^= 1;
       ctx->parity ^= 1;
       ctx->step += 1;
     }
-  } else if (c.opt_policy == CULBM_OPT_MIXED) {
-    // two steps per launch across the passes of innerLoop steps (the bits do
-    // not depend on the grouping), one plain step for an odd remainder
-    return fused_pass<S>(ctx, nsteps);
   } else {
     int32_t left = nsteps;
     while (left > 0) {
@@ -760,6 +786,90 @@ int32_t auto_depth(const culbm_ctx* ctx) {
   return std::max(2, std::min(d, nz));
 }
 
+// Launch shape of k_fused2, and whether it is the faster way to take two pull
+// steps, from a cost model in microseconds.
+//
+// A workgroup fills a CU, so `rounds` of them run one after the other, each
+// zchunk + 2 planes long (two A planes are recomputed per chunk) at a cost per
+// plane that follows the waves of A and B cells on the fullest of the CU's four
+// SIMDs; its memory costs what it writes and the rows or lines of halo it reads,
+// and the two overlap (a 3-norm).  Candidates: the domain's width in equal tile
+// columns, as it falls or rounded up to 32 cells, as many rows as fit 1024
+// threads, and up to 64 chunks.  Fitted to 19 domains from 64^3 to 384x384x200,
+// 449 tile and chunk choices per storage (0.07-0.13 rms of the logarithm): the
+// pick costs 0.6 % (16-bit), 1.5 % (FP32) and 1.3 %
+// (stochastic rounding) over the best measured one on average.  Some of them,
+// in MLUPS: FP32 at 288x272x280 96x8 (43.5k; 48x17 41.7k, 64x13 40.9k), at
+// 203x170x119 102x7 (34.9k; 96x8 27.4k), at 48x200x150 48x17 (34.7k; 64x13
+// 33.6k); FP16 at 33x270x280 33x27 (51.9k; 64x13 34.3k).
+//
+// A plain step costs 3.3 us and a rate that steps down once its two buffers
+// pass the cache.  Measured either side of the line, two steps per launch
+// against plain steps: FP32 at 80^3 25.6k vs 28.0k MLUPS, at 96^3 36.5k vs
+// 28.7k; FP16 at 107x109x78 48.3k vs 50.6k, at 150x220x90 50.5k vs 44.5k; FP16
+// with stochastic rounding at 203x170x119 43.2k vs 45.0k, at 192x160x176 49.0k
+// vs 46.0k.
+FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
+  const culbm_config& c = ctx->cfg;
+  const bool wide = ctx->bpp == 4;
+  const double cells = double(c.nx) * c.ny * c.nz;
+  // per plane of a workgroup: fixed, per wave of A and of B cells on a SIMD
+  const double fix = wide ? 0.0 : (ctx->sr ? 1.37 : 0.17), wa = wide ? 0.66 : (ctx->sr ? 0.46 : 0.68),
+               wb = wide ? 0.98 : (ctx->sr ? 0.65 : 0.45);
+  // per 128 bytes written, the share of them that an unaligned tile row writes
+  // once more, and per row of A cells: fixed, per line read
+  const double write = 128e-6 * (wide ? 0.37 : (ctx->sr ? 0.669 : 0.544));
+  const double edge = wide ? 0.38 : (ctx->sr ? 0.08 : 0.11);
+  const double row = 128e-6 * (wide ? 0.0 : (ctx->sr ? 0.020 : 0.037)), line = 128e-6 * (wide ? 0.03 : 0.0);
+  const bool given = c.opt_policy == CULBM_OPT_MIXED && c.wave_depth > 0;
+  FusedPlan best;
+  double best_us = 0.0;
+  const int64_t least = (int64_t(c.nx) + kFusedBlock / 3 - 3) / (kFusedBlock / 3 - 2);  // columns of three A rows
+  for (int64_t m = least; m == least || (m < least + 48 && (c.nx + m - 1) / m >= 24); ++m) {
+    const int even = int((c.nx + m - 1) / m);
+    for (int tx : {even, int(round_up(even, 32))}) {
+      const int rows = std::min(kFusedBlock / (tx + 2), kFusedRows) - 2;
+      if (rows < 1) continue;
+      FusedPlan p;
+      p.tx = tx;
+      p.tiles_x = int32_t((int64_t(c.nx) + tx - 1) / tx);
+      const int64_t even_y = (int64_t(c.ny) + rows - 1) / rows;
+      p.ty = int32_t((c.ny + even_y - 1) / even_y);
+      p.tiles_y = int32_t((int64_t(c.ny) + p.ty - 1) / p.ty);
+      const double tiles = double(p.tiles_x) * p.tiles_y;
+      const double plane_us = fix + wa * std::ceil((tx + 2) * (p.ty + 2) / 256.0) + wb * std::ceil(tx * p.ty / 256.0);
+      const bool aligned = tx * ctx->bpp % 64 == 0 && c.nx * ctx->bpp % 64 == 0;
+      const double out = double(p.tiles_x) * c.ny * c.nz * (tx * ctx->bpp / 128.0 + (aligned ? 0.0 : edge));
+      const double reads = tiles * (p.ty + 2) * (row + line * ((tx + 2) * ctx->bpp / 128.0 + 1.0));
+      for (int n = 1; n <= (given ? 1 : std::min(64, c.nz)); ++n) {
+        p.zchunk = given ? std::min(c.wave_depth, c.nz) : int32_t((int64_t(c.nz) + n - 1) / n);
+        p.nchunk = int32_t((int64_t(c.nz) + p.zchunk - 1) / p.zchunk);
+        const double march = std::ceil(tiles * p.nchunk / ncu) * (p.zchunk + 2) * plane_us;
+        const double mem = 27.0 * (write * out + reads * (c.nz + 2.0 * p.nchunk));
+        const double us = std::cbrt(march * march * march + mem * mem * mem);
+        if (best.nchunk == 0 || us < best_us * (1.0 - 1e-9)) {
+          best = p;
+          best_us = us;
+        }
+      }
+    }
+  }
+  const bool cached = 2.0 * 27.0 * ctx->bpp * cells < 240e6;
+  const double cell_us = 1e-6 * (wide ? (cached ? 30.0 : 42.0) : (cached ? 18.0 : 21.6));
+  // a launch's own start and fill count where it is short; ties go to the plain steps
+  best.pays = best_us + (wide ? 2.0 : 6.0) < (ctx->sr ? 1.0 : (c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95)) * 2.0 * (3.3 + cells * cell_us);
+  return best;
+}
+
+// Pull steps in pairs?  The mixed policy's form, except where it leaves the
+// depth to the library and plain steps are faster.
+bool fused_pairs(const culbm_ctx* ctx) {
+  const culbm_config& c = ctx->cfg;
+  if (ctx->inplace || !fused_scale_ok(ctx)) return false;
+  if (c.opt_policy != CULBM_OPT_MIXED) return false;
+  return c.wave_depth > 0 || ctx->fused.pays;
+}
+
 // Moment sums: at most kSumParts workgroups, each writing one partial of the
 // four sums, then the four totals after them: the work array holds
 // 4 * kSumParts + 4 doubles whatever the domain.
@@ -902,44 +1012,10 @@ int culbm_create(const culbm_config* cfg, culbm_ctx** out) {
     ctx->wave_depth = c.wave_depth > 0 ? std::min(c.wave_depth, c.nz) : auto_depth(ctx);
   }
   {
-    // k_fused2's launch shape, for the mixed policy and for the adjoint's
-    // forward sweeps: z-chunks per tile column balance the workgroup count over
-    // the resident workgroup slots against the two extra A planes a chunk
-    // recomputes
     int ncu = 256;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, c.device) == hipSuccess) ncu = prop.multiProcessorCount;
-    int per_cu = 1;
-    by_storage(c.storage, [&](auto s) {
-      using S = decltype(s);
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&k_fused2<S, false>),
-                                                       FusedShape<S::kBytes>::BLOCK, 0) != hipSuccess)
-        per_cu = 1;
-      return 0;
-    });
-    const int slots = ncu * std::max(per_cu, 1);
-    const int ftx = ctx->bpp == 4 ? FusedShape<4>::TX : FusedShape<2>::TX;
-    const int fty = ctx->bpp == 4 ? FusedShape<4>::TY : FusedShape<2>::TY;
-    ctx->tiles_x = (c.nx + ftx - 1) / ftx;
-    ctx->tiles_y = (c.ny + fty - 1) / fty;
-    const double tiles = double(ctx->tiles_x) * ctx->tiles_y;
-    if (c.opt_policy == CULBM_OPT_MIXED && c.wave_depth > 0) {
-      ctx->fzchunk = std::min(c.wave_depth, c.nz);
-    } else {
-      double best = 1e30;
-      for (int n = 1; n <= std::min(64, c.nz); ++n) {
-        const int len = (c.nz + n - 1) / n;
-        const double wgs = tiles * n;
-        const double rounds = std::ceil(wgs / slots);
-        const double cost = rounds / (wgs / slots) * (1.0 + 2.0 / len);
-        if (cost < best - 1e-9) {
-          best = cost;
-          ctx->fzchunk = len;
-        }
-      }
-    }
-    ctx->nchunk = (c.nz + ctx->fzchunk - 1) / ctx->fzchunk;
-    if (c.opt_policy == CULBM_OPT_MIXED) ctx->wave_depth = ctx->fzchunk;  // reported as the depth
+    ctx->fused = fused_plan(ctx, ncu);
   }
 
   // reference defaults: all FLUID + DUMP, rho 1, u 0, rest populations
@@ -1218,14 +1294,17 @@ int culbm_get_info(culbm_ctx* ctx, culbm_info* info) {
   std::memset(info, 0, sizeof(*info));
   info->step = ctx->step;
   info->device_bytes = ctx->device_bytes;
-  info->wave_depth = ctx->wave_depth;
+  const bool pairs = fused_pairs(ctx);
+  info->wave_depth = blocked(ctx->cfg) && (pairs || ctx->cfg.opt_policy == CULBM_OPT_MIXED) ? ctx->fused.zchunk : ctx->wave_depth;
   info->bytes_per_pop = ctx->bpp;
   info->storage_scale = ctx->scale;
   const culbm_config& c = ctx->cfg;
   if (!blocked(c)) {
     info->launches_per_pass = 1;
-  } else if (c.opt_policy == CULBM_OPT_MIXED) {
+  } else if (pairs) {
     info->launches_per_pass = (c.inner_loop + 1) / 2;  // two steps per launch (pairs run across passes)
+  } else if (c.opt_policy == CULBM_OPT_MIXED) {
+    info->launches_per_pass = c.inner_loop;
   } else {
     int32_t cnt = 0;
     for_each_wave_launch(c.nz, ctx->wave_depth, c.inner_loop, [&](int32_t, int32_t, int32_t) {

@@ -45,13 +45,11 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nblk) {
 // measured; 8 and 16 lead in every form).
 constexpr uint32_t kXcdGroup = 8;
 
-template <uint32_t RUN = kXcdGroup>
-__device__ __forceinline__ uint32_t xcd_group(uint32_t b, uint32_t nblk) {
-  constexpr uint32_t G = 8u * RUN;
-  const uint32_t sg = b / G;
-  if ((sg + 1) * G > nblk) return b;
-  const uint32_t r = b - sg * G;
-  return sg * G + (r & 7u) * RUN + (r >> 3);
+__device__ __forceinline__ uint32_t xcd_group(uint32_t b, uint32_t nblk, uint32_t run = kXcdGroup) {
+  const uint32_t g = 8u * run, sg = b / g;
+  if ((sg + 1) * g > nblk) return b;
+  const uint32_t r = b - sg * g;
+  return sg * g + (r & 7u) * run + (r >> 3);
 }
 
 // The workgroup order of a cell launch, chosen by the host per launch (a.order):
@@ -488,250 +486,6 @@ __global__ __launch_bounds__(kBlock) void k_twist(const StepArgs a) {
   const uint32_t fl = a.sflag[k.c];
   update_cell(fl, a, k.c, q, f);
   if (fl & kStore) twist_store_all<S, P, SR, !XR>(a, k, a.dst, f, make_encoder<S, SR>(a, k.c, a.state));
-}
-
-// ---------------------------------------------------------------------------
-// Two steps per launch with the intermediate populations kept in LDS (the
-// mixed L1/L2 blocking of the reference, HALO_BLOCKING_L1L2,
-// kernel.cu:138-329, redesigned for the 160 KB LDS of a gfx950 CU).
-//
-// A workgroup owns a TX x TY tile of cells and marches along z over a chunk
-// of planes.  For each plane it computes the first step on the tile plus a
-// one-cell xy halo ("A" cells, pulled from src in HBM) into a 3-plane LDS ring,
-// then the second step of the tile ("B" cells, pulled from the ring) into dst.
-// HBM sees the first step's reads (tile + halo) and the second step's writes
-// only.  The intermediate is kept in the storage format, exactly as a plain
-// step would have stored it, so two fused steps equal two plain steps bit for
-// bit.  A cell without STORE keeps its populations in both buffers (see
-// culbm_set_state), so its intermediate value is its src value.
-
-// Tile of a workgroup per storage width: TX x TY B cells, (TX+2)(TY+2) A cells
-// (the tile and a one-cell xy halo), one thread per A cell.
-template <int BYTES>
-struct FusedTile;
-template <>
-struct FusedTile<4> {
-  static constexpr int TX = 32, TY = 16, BLOCK = 640;  // 612 A cells, ten waves
-};
-template <>
-struct FusedTile<2> {
-  static constexpr int TX = 96, TY = 8, BLOCK = 1024;  // 980 A cells, sixteen waves
-};
-template <int BYTES>
-struct FusedShape : FusedTile<BYTES> {
-  using Base = FusedTile<BYTES>;
-  static constexpr int AX = Base::TX + 2, AY = Base::TY + 2, A = AX * AY;
-  static_assert(A <= Base::BLOCK && Base::BLOCK % 64 == 0 && Base::BLOCK <= 1024, "one A cell per thread");
-};
-
-struct FusedArgs {
-  StepArgs a;
-  int32_t tiles_x, tiles_y;
-  int32_t zchunk;  // B planes per workgroup
-  int32_t nchunk;
-};
-
-// LDS of one workgroup.  A plane's first-step populations are grouped by c_z:
-// the c_z = +1 group is read by the B step of the next plane, the c_z = 0 group
-// by the same plane, the c_z = -1 group by the previous plane, so the groups
-// live 3, 2 and 1 plane(s): 54 values per A cell instead of 81.
-template <class T>
-struct FusedRing {
-  using F = FusedShape<sizeof(T)>;
-  T up[3][9][F::A];  // directions 18..26 (c_z = +1), slot = plane % 3
-  T mid[2][9][F::A]; // directions 9..17 (c_z = 0), slot = plane % 2
-  T dn[9][F::A];     // directions 0..8 (c_z = -1), the latest plane
-  uint8_t fl[2][F::A];  // step bits of the A cells, slot = plane % 2 (the B step's flags)
-  float eq[2][2][F::TY][4];  // EQU inputs of the B cells on the low / high x face, slot = plane % 2
-};
-
-// Pulled (not yet updated) populations of one A cell, gathered a plane ahead
-// so the HBM latency overlaps the previous plane's second step.
-struct APending {
-  float f[27];
-  uint8_t fl;  // kept 8-bit: a widened copy across the loop would wait for every load
-  uint32_t c;
-  bool ok;
-};
-
-template <class S>
-// Every lane gathers, at a position clamped into the domain (the caller clamps
-// the plane), and only q.ok tells whether the cell is used: loads issued on
-// every path let the compiler wait for exactly one gather while the next one
-// is still in flight, instead of for every outstanding load.
-__device__ __forceinline__ void fused_a_gather(const StepArgs& a, int32_t x0, int32_t y0, int ac,
-                                               int32_t p, APending& q) {
-  using F = FusedShape<sizeof(typename S::T)>;
-  const int32_t gx = x0 - 1 + ac % F::AX, gy = y0 - 1 + ac / F::AX;
-  q.ok = ac < F::A && gx >= 0 && gx < a.nx && gy >= 0 && gy < a.ny;
-  Cell k;
-  k.x = min(max(gx, 0), a.nx - 1);
-  k.y = min(max(gy, 0), a.ny - 1);
-  k.z = p;
-  k.c = (uint32_t(p) * uint32_t(a.ny) + uint32_t(k.y)) * uint32_t(a.nx) + uint32_t(k.x);
-  k.l = k.c;
-  q.c = k.c;
-  make_gather<S>(a, k, a.src).template run<0>(q.f);
-  q.fl = a.sflag[k.c];
-}
-
-template <class S, bool SR, int I>
-__device__ __forceinline__ void encode_all(const float* f, typename S::T* v, const Encoder<S, SR>& e) {
-  v[I] = e.template get<I>(f[I]);
-  if constexpr (I < 26) encode_all<S, SR, I + 1>(f, v, e);
-}
-
-// First step of a gathered A cell into the ring: a plain pull update (the state
-// numbered a.state), or the cell's own populations when it has no STORE.
-template <class S, bool SR>
-__device__ __forceinline__ void fused_a_finish(const StepArgs& a, int ac, int32_t p, APending& q,
-                                               FusedRing<typename S::T>& r) {
-  using T = typename S::T;
-  if (!q.ok) return;
-  // An x-face EQU cell loads its inputs here, once its flag is known (carrying
-  // them in the two pending sets would spill registers in FP32), and passes
-  // them to the second step through LDS, where a load would wait for the
-  // gathers in flight.
-  EquIn qe;
-  const uint32_t gx = q.c % uint32_t(a.nx);
-  qe.ok = (q.fl & kEqu) && (gx == 0 || gx == uint32_t(a.nx - 1));
-  qe.rho = qe.vx = qe.vy = qe.vz = 0.0f;
-  if (qe.ok) {
-    qe.rho = a.rho[q.c];
-    qe.vx = a.vx[q.c];
-    qe.vy = a.vy[q.c];
-    qe.vz = a.vz[q.c];
-  }
-  update_cell(q.fl, a, q.c, qe, q.f);
-  T v[27];
-  if (q.fl & kStore) {
-    encode_all<S, SR, 0>(q.f, v, make_encoder<S, SR>(a, q.c, a.state));
-  } else {
-    constexpr uint32_t B = sizeof(T);
-    const char* src = static_cast<const char*>(a.src);
-#pragma unroll
-    for (int i = 0; i < 27; ++i) v[i] = ld_at<T>(src + i * (a.dstride * B), q.c * B);
-  }
-  const int su = p % 3, sm = p % 2;
-  r.fl[sm][ac] = uint8_t(q.fl);
-  // EQU inputs of the x-face cells among the B cells, for the second step
-  const int ly = ac / FusedShape<sizeof(T)>::AX - 1;
-  if (qe.ok && ly >= 0 && ly < FusedShape<sizeof(T)>::TY) {
-    float* d = r.eq[sm][gx == 0 ? 0 : 1][ly];
-    d[0] = qe.rho;
-    d[1] = qe.vx;
-    d[2] = qe.vy;
-    d[3] = qe.vz;
-  }
-#pragma unroll
-  for (int j = 0; j < 9; ++j) {
-    r.dn[j][ac] = v[j];
-    r.mid[sm][j][ac] = v[9 + j];
-    r.up[su][j][ac] = v[18 + j];
-  }
-}
-
-template <class S, bool SR>
-// At most 168 VGPRs (three waves per SIMD), room for the ten waves of an FP32
-// workgroup; the sixteen waves of a 16-bit workgroup bound it to 128.
-__global__ __launch_bounds__(FusedShape<S::kBytes>::BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void k_fused2(
-    const FusedArgs fa) {
-  using T = typename S::T;
-  using F = FusedShape<sizeof(T)>;
-  __shared__ FusedRing<T> r;
-  const uint32_t ntile = uint32_t(fa.tiles_x) * fa.tiles_y * fa.nchunk;
-  // runs of 16 tiles per XCD, tiles in x-major order: x neighbours, whose
-  // halos share lines, mostly run on one XCD at the same time.  At 288x272x280,
-  // against dispatching the x-face tile columns first: FP32 +2.6 % (runs of 8:
-  // +2.3 %); against runs of 8: FP16 +0.4 %.
-  const uint32_t w = xcd_group<16>(blockIdx.x, ntile);
-  const int32_t tx = int32_t(w % uint32_t(fa.tiles_x));
-  const int32_t ty = int32_t((w / uint32_t(fa.tiles_x)) % uint32_t(fa.tiles_y));
-  const int32_t zc = int32_t(w / (uint32_t(fa.tiles_x) * fa.tiles_y));
-  const int32_t x0 = tx * F::TX, y0 = ty * F::TY;
-  const int32_t nx = fa.a.nx, ny = fa.a.ny, nz = fa.a.nz;
-  const int32_t zs = zc * fa.zchunk, ze = min(nz, zs + fa.zchunk);
-  const int t = threadIdx.x;
-  const bool a_ok = t < F::A;
-
-  // A planes gathered ahead of their first step: two for FP32 (the gather
-  // latency then spans two planes' B steps), one for 16-bit storage
-  constexpr int kAhead = sizeof(T) == 4 ? 2 : 1;
-  APending q0, q1;
-  q0.ok = false;
-  q1.ok = false;
-  // prologue: A planes zs-1 (if any) and zs, then the gathers of planes zs+1 (, zs+2)
-  for (int32_t p = max(zs - 1, 0); p <= zs; ++p) {
-    fused_a_gather<S>(fa.a, x0, y0, t, p, q0);
-    if (a_ok) fused_a_finish<S, SR>(fa.a, t, p, q0, r);
-    __syncthreads();  // the dn group of plane zs-1 is overwritten by plane zs
-  }
-  // planes past the chunk (or the domain) are gathered too, clamped, and unused
-  fused_a_gather<S>(fa.a, x0, y0, t, min(zs + 1, nz - 1), q0);
-  if (kAhead == 2) fused_a_gather<S>(fa.a, x0, y0, t, min(zs + 2, nz - 1), q1);
-
-  const int bx = t % F::TX, by = t / F::TX;
-  const int32_t gx = x0 + bx, gy = y0 + by;
-  const bool b_ok = t < F::TX * F::TY && gx < nx && gy < ny;
-  // local A coordinates of the (clamped) source columns
-  const int lxm = gx == 0 ? bx + 1 : bx, lxp = gx == nx - 1 ? bx + 1 : bx + 2;
-  const int lym = gy == 0 ? by + 1 : by, lyp = gy == ny - 1 ? by + 1 : by + 2;
-  const uint32_t cxy = uint32_t(gy) * uint32_t(nx) + uint32_t(gx), pl = uint32_t(nx) * uint32_t(ny);
-  const int bc = (by + 1) * F::AX + bx + 1;  // the B cell among the A cells
-  // B plane z; q holds the gathered A plane z+1 and receives A plane z+1+kAhead.
-  // The B step issues no global load: its flag byte comes from the A step's
-  // copy in LDS, so no wait on a global load can hold back the A gathers
-  // still in flight (the counter of vector memory operations is in order).
-  auto plane = [&](int32_t z, APending& q) {
-    if (a_ok && z + 1 < nz) fused_a_finish<S, SR>(fa.a, t, z + 1, q, r);
-    fused_a_gather<S>(fa.a, x0, y0, t, min(z + 1 + kAhead, nz - 1), q);
-    __syncthreads();
-    if (b_ok) {
-      // c_z = +1 pulls from plane z-1 (clamped to z), c_z = -1 from z+1 (the
-      // dn group still holds plane z when z is the last plane)
-      const int su = (z == 0 ? z : z - 1) % 3, sm = z % 2;
-      float f[27];
-#pragma unroll
-      for (int i = 0; i < 27; ++i) {
-        const int cx = cx_of(i), cy = cy_of(i), cz = cz_of(i);
-        const int lx = cx == 1 ? lxm : (cx == -1 ? lxp : bx + 1);
-        const int ly = cy == 1 ? lym : (cy == -1 ? lyp : by + 1);
-        const int a = ly * F::AX + lx;
-        const T v = cz == 1 ? r.up[su][i - 18][a] : (cz == 0 ? r.mid[sm][i - 9][a] : r.dn[i][a]);
-        f[i] = S::dec(v, fa.a.inv_scale);
-      }
-      Cell k;
-      k.x = gx;
-      k.y = gy;
-      k.z = z;
-      k.c = uint32_t(z) * pl + cxy;
-      k.l = k.c;
-      const uint32_t fl = r.fl[z % 2][bc];
-      EquIn e;
-      e.ok = gx == 0 || gx == nx - 1;
-      const float* q4 = r.eq[z % 2][gx == 0 ? 0 : 1][by];
-      e.rho = q4[0];
-      e.vx = q4[1];
-      e.vy = q4[2];
-      e.vz = q4[3];
-      update_cell(fl, fa.a, k.c, e, f);
-      if (fl & kStore)  // the second step produces state a.state + 1
-        store_plain_all<S, SR>(fa.a, k, fa.a.dst, f, make_encoder<S, SR>(fa.a, k.c, fa.a.state + 1));
-    }
-    __syncthreads();
-  };
-  int32_t z = zs;
-  if constexpr (kAhead == 2) {
-    // both halves on every trip (an odd last plane follows the loop): the
-    // compiler then counts the other set's gather as in flight at every wait
-    for (; z + 1 < ze; z += 2) {
-      plane(z, q0);
-      plane(z + 1, q1);
-    }
-    if (z < ze) plane(z, q0);
-  } else {
-    for (; z < ze; ++z) plane(z, q0);
-  }
 }
 
 // ---------------------------------------------------------------------------

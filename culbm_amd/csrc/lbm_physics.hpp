@@ -43,9 +43,13 @@ struct Moments {
 
 // calcRhoU<27>: rho = (1+f0) + (f1+f2) + ... + (f25+f26) left to right;
 // u = (sum of c-signed pairs) * (1/rho).
-__device__ __forceinline__ Moments moments(const float* f) {
+//
+// `one`: the populations' unit.  Populations multiplied by a power of two s
+// (one = s) give s rho and the same u: scaling by s commutes with every
+// rounding here as long as neither side leaves the normal range.
+__device__ __forceinline__ Moments moments(const float* f, float one = 1.0f) {
   Moments m;
-  float rho = 1.0f + f[0];
+  float rho = one + f[0];
 #pragma unroll
   for (int k = 1; k < 27; k += 2) rho = rho + (f[k] + f[k + 1]);
   const float inv = 1.0f / rho;
@@ -95,9 +99,10 @@ struct EqTerms {
   float rws, rwe, rwc, mws, mwe, mwc;
 };
 
-__device__ __forceinline__ void eq_terms(float rho, float vx, float vy, float vz, EqTerms& e) {
+// With rho in units of `one` the equilibrium of these terms is in them too.
+__device__ __forceinline__ void eq_terms(float rho, float vx, float vy, float vz, EqTerms& e, float one = 1.0f) {
   e.rho = rho;
-  e.rhom1 = rho - 1.0f;
+  e.rhom1 = rho - one;
   e.c3 = -3.0f * (vx * vx + vy * vy + vz * vz);
   vx *= 3.0f;
   vy *= 3.0f;
