@@ -861,13 +861,14 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   return best;
 }
 
-// Pull steps in pairs?  The mixed policy's form, except where it leaves the
-// depth to the library and plain steps are faster.
+// Pull steps in pairs?  Every pull policy gives the same bits, so a context
+// that leaves the blocking to the library (no explicit depth) takes the fastest
+// form; an explicit depth asks for that policy's own schedule.
 bool fused_pairs(const culbm_ctx* ctx) {
   const culbm_config& c = ctx->cfg;
   if (ctx->inplace || !fused_scale_ok(ctx)) return false;
-  if (c.opt_policy != CULBM_OPT_MIXED) return false;
-  return c.wave_depth > 0 || ctx->fused.pays;
+  if (c.opt_policy == CULBM_OPT_MIXED && c.wave_depth > 0) return true;
+  return ctx->fused.pays && (!blocked(c) || c.wave_depth == 0);
 }
 
 // Moment sums: at most kSumParts workgroups, each writing one partial of the
