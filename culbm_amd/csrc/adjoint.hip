@@ -67,8 +67,9 @@ __device__ __forceinline__ void adj_gather_consumers(const AdjArgs& j, const Cel
                                                      const float* mu, float* lo) {
   const StepArgs& a = j.a;
   const char* base = reinterpret_cast<const char*>(mu);
-  const int64_t dsb = a.dstride * 4;
-  const uint32_t lb = k.l * 4u;
+  int64_t dsb = a.dstride * 4;
+  uint32_t lb = k.l * 4u;
+  asm volatile("" : "+s"(dsb), "+v"(lb));  // see k_adjoint
   const ConsumerOffsets o = consumer_offsets(a, k);
 #pragma unroll
   for (int i = 0; i < 27; ++i) {
@@ -77,6 +78,9 @@ __device__ __forceinline__ void adj_gather_consumers(const AdjArgs& j, const Cel
     lo[i] = (o.vx[cx + 1] && o.vy[cy + 1] && o.vz[cz + 1]) ? v : 0.0f;
   }
   if (!o.vx[0] || !o.vx[2]) {  // x face: the cell itself consumes along x
+    int64_t dsb = a.dstride * 4;
+    uint32_t lb = k.l * 4u;
+    asm volatile("" : "+s"(dsb), "+v"(lb));
     // every lane of the wave loads (all addresses are in the domain) and keeps
     // the value where it applies: one wait for the batch instead of one
     // round trip per conditional load
@@ -99,6 +103,9 @@ __device__ __forceinline__ void adj_gather_consumers(const AdjArgs& j, const Cel
     // in three batches of nine directions (one c_z each), loads first
 #pragma unroll
     for (int g = 0; g < 3; ++g) {
+      int64_t dsb = a.dstride * 4;
+      uint32_t lb = k.l * 4u;
+      asm volatile("" : "+s"(dsb), "+v"(lb));
       float e[9][6];
 #pragma unroll
       for (int i = 9 * g; i < 9 * g + 9; ++i) {
@@ -171,17 +178,21 @@ __device__ __forceinline__ float umu(const LamMoments& m, float ux, float uy, fl
 // With bb the collision acts on the bounced state h'_i = h_{26-i}: the same rho,
 // the opposite momentum, and lam . h' = sum lam_i h_{26-i}, so h is never permuted.
 __device__ __forceinline__ float adj_collide(float inv_tau, const float* h, float* lam, bool bb) {
-  float rho = 1.0f, mx = 0.0f, my = 0.0f, mz = 0.0f, l0 = 0.0f, l1 = 0.0f;
+  float rho = 1.0f, mx = 0.0f, my = 0.0f, mz = 0.0f, lh = 0.0f;
 #pragma unroll
   for (int i = 0; i < 27; ++i) {
     rho += h[i];
     if (cx_of(i) != 0) mx += cx_of(i) > 0 ? h[i] : -h[i];
     if (cy_of(i) != 0) my += cy_of(i) > 0 ? h[i] : -h[i];
     if (cz_of(i) != 0) mz += cz_of(i) > 0 ? h[i] : -h[i];
-    l0 += lam[i] * h[i];
-    l1 += lam[i] * h[26 - i];
+    lh += lam[i] * h[i];
   }
-  const float lh = bb ? l1 : l0;
+  if (__ballot(bb)) {  // a wave with a cell that bounces and collides
+    float l1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 27; ++i) l1 += lam[i] * h[26 - i];
+    if (bb) lh = l1;
+  }
   const float inv = bb ? -1.0f / rho : 1.0f / rho;
   const float ux = mx * inv, uy = my * inv, uz = mz * inv;
   const float u2 = ux * ux + uy * uy + uz * uz;
@@ -234,11 +245,18 @@ __device__ __forceinline__ double block_sum(double v) {
   return s;
 }
 
-// One reverse step: mu^t from mu^{t+1} and f^t.  Both gathers are in bounds for every cell, so they are issued
-// before the flag arrives.  With wobj the objective's term is added to mu^t.
+// One reverse step: mu^t from mu^{t+1} and f^t.  Both gathers are in bounds for
+// every cell, so they are issued before the flag arrives.  With wobj the
+// objective's term is added to mu^t.
+//
+// Bound by its bytes: 333 counted per cell, 144 us at 128^3, 4.86 TB/s.  Each
+// batch of loads or stores takes the direction stride and the lane offset anew
+// (the empty asm statements): held over the kernel, the 81 direction bases
+// spilled 48 scalar registers to vector lanes and most addresses were formed in
+// vector registers (147 us, 120 VGPRs; now 102, no spills).
 template <class S>
 // Four waves per SIMD: the batched face loads would otherwise take the register
-// count past 128.
+// count past 128.  Five (96 VGPRs, 7 spilled) run at the same rate.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint(
     const AdjArgs j) {
   const StepArgs& a = j.a;
@@ -277,7 +295,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       else if (!(fl & kLoad))
         clear(h);
       if (fl & kCollide) dtau = adj_collide(a.inv_tau, h, lam, bb);
-      if (bb) bounce_back(lam);
+      if (bb) fused_bounce_back(lam);
       if (fl & kEqu) {
         float g4[4];
         adj_feq_inputs(q.rho, q.vx, q.vy, q.vz, lam, g4);
@@ -299,8 +317,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       for (int i = 0; i < 27; ++i) lam[i] += wq * (float(cx_of(i)) - wux);
     }
     char* out = reinterpret_cast<char*>(j.mu_out);
+    int64_t dsb = a.dstride * 4;
+    uint32_t lb = k.l * 4u;
+    asm volatile("" : "+s"(dsb), "+v"(lb));
 #pragma unroll
-    for (int i = 0; i < 27; ++i) st_at<float>(out + i * (a.dstride * 4), k.l * 4u, lam[i]);
+    for (int i = 0; i < 27; ++i) st_at<float>(out + i * dsb, lb, lam[i]);
   }
   // one accumulator per block of cells (not per hardware workgroup), so the
   // fixed-order host sum does not depend on the workgroup order
