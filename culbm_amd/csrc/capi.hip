@@ -25,6 +25,7 @@ using namespace culbm;
 // and z chunks; `pays`: two steps in one launch beat two plain steps.
 struct FusedPlan {
   int32_t tx = 0, ty = 0, tiles_x = 0, tiles_y = 0, zchunk = 0, nchunk = 0;
+  bool nt = false;  // non-temporal stores
   bool pays = false;
 };
 
@@ -572,12 +573,15 @@ void launch_fused(const culbm_ctx* ctx, const StepArgs& a) {
   const dim3 grid(uint32_t(p.tiles_x) * uint32_t(p.tiles_y) * uint32_t(p.nchunk));
   const dim3 block(uint32_t(round_up(int64_t(p.tx + 2) * (p.ty + 2), 64)));
   if constexpr (S::kBytes == 2) {
-    if (ctx->sr) {
-      hipLaunchKernelGGL((k_fused2<S, true>), grid, block, 0, ctx->stream, fa);
-      return;
-    }
+    if (ctx->sr)
+      hipLaunchKernelGGL((k_fused2<S, true, false>), grid, block, 0, ctx->stream, fa);
+    else
+      hipLaunchKernelGGL((k_fused2<S, false, false>), grid, block, 0, ctx->stream, fa);
+  } else if (p.nt) {
+    hipLaunchKernelGGL((k_fused2<S, false, true>), grid, block, 0, ctx->stream, fa);
+  } else {
+    hipLaunchKernelGGL((k_fused2<S, false, false>), grid, block, 0, ctx->stream, fa);
   }
-  hipLaunchKernelGGL((k_fused2<S, false>), grid, block, 0, ctx->stream, fa);
 }
 
 bool fused_pairs(const culbm_ctx* ctx);
@@ -1019,6 +1023,12 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   }
   const bool cached = 2.0 * 27.0 * ctx->bpp * cells < 240e6;
   const double cell_us = 1e-6 * (wide ? (cached ? 30.0 : 42.0) : (cached ? 18.0 : 21.6));
+  // Non-temporal stores leave the L2 to the halo lines: FP32 rows of whole 64-byte
+  // blocks whose buffers pass the cache gain (MLUPS without and with: 128^3 32.6k,
+  // 34.1k; 192x160x176 38.9k, 39.7k; 256^3 37.6k, 40.3k; 288x272x280 42.6k, 43.2k);
+  // blocks shared by two tiles are then written twice (203x170x119 34.9k, 25.3k),
+  // cached buffers miss (96^3 36.6k, 34.0k), and 16-bit rows go either way.
+  best.nt = wide && !cached && c.nx % 16 == 0 && best.tx % 16 == 0;
   // a launch's own start and fill count where it is short; ties go to the plain steps
   best.pays = best_us + (wide ? 2.0 : 6.0) < (ctx->sr ? 1.0 : (c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95)) * 2.0 * (3.3 + cells * cell_us);
   return best;

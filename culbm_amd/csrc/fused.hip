@@ -25,7 +25,8 @@
 // same +4 %, computing in units of the storage scale +8 %, one barrier per plane
 // +6 %.  Measured and left out: gathers two planes ahead (fewer waves or spills:
 // FP32 64x8 34.5k), two workgroups of 32x12 per CU (29.5k), releasing the LDS
-// before the second step's arithmetic (spills, 35.8k), non-temporal stores (equal).
+// before the second step's arithmetic (spills, 35.8k), non-temporal loads (30.3k;
+// of the rows no other tile reads only, equal).
 //
 // The intermediate is kept in the storage format, exactly as a plain
 // step would have stored it, so two fused steps equal two plain steps bit for
@@ -269,13 +270,18 @@ __device__ __forceinline__ void fused_first(const StepArgs& a, int ac, const Fus
   if (!(q.fl & kStore)) fused_keep<S>(a, zc, k.c, [&](int i, T x) { (i < 18 ? r.lo[ll][i] : r.up[sl][i - 18])[ac] = x; });
 }
 
-template <class S, int I>
+template <class S, bool NT, int I>
 __device__ __forceinline__ void fused_store_dir(char* base, int64_t dsb, uint32_t lb, const typename S::T* v) {
-  st_at<typename S::T>(base + I * dsb, lb, v[I]);
-  if constexpr (I < 26) fused_store_dir<S, I + 1>(base, dsb, lb, v);
+  using T = typename S::T;
+  if constexpr (NT)
+    __builtin_nontemporal_store(v[I], reinterpret_cast<T*>(base + I * dsb + lb));
+  else
+    st_at<T>(base + I * dsb, lb, v[I]);
+  if constexpr (I < 26) fused_store_dir<S, NT, I + 1>(base, dsb, lb, v);
 }
 
-template <class S, bool SR>
+// NT: non-temporal stores of the second step (fused_plan says where).
+template <class S, bool SR, bool NT>
 __global__ __launch_bounds__(kFusedBlock) void k_fused2(const FusedArgs fa) {
   using T = typename S::T;
   using P = FusedPlane<T>;
@@ -407,7 +413,7 @@ __global__ __launch_bounds__(kFusedBlock) void k_fused2(const FusedArgs fa) {
         uint32_t lb = cxy * uint32_t(sizeof(T));
         asm volatile("" : "+v"(lb));
         char* dst = static_cast<char*>(a.dst) + zc * sizeof(T);
-        fused_store_dir<S, 0>(dst, dsb, lb, v);
+        fused_store_dir<S, NT, 0>(dst, dsb, lb, v);
         if (!(fl & kStore)) {  // dst keeps its bits
           T* own = static_cast<T*>(a.dst) + zc + cxy;
           fused_keep<S>(a, zc, cxy, [&](int i, T x) { own[i * a.dstride] = x; });
