@@ -1021,7 +1021,9 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
       }
     }
   }
-  const bool cached = 2.0 * 27.0 * ctx->bpp * cells < 240e6;
+  // (at 226 MB, FP16 128^3, plain steps ran 46k or 54k MLUPS from one context to
+  // the next and the pairs 53k to 55k; with stochastic rounding 45k or 52k, and 45k)
+  const bool cached = 2.0 * 27.0 * ctx->bpp * cells < (ctx->sr ? 240e6 : 210e6);
   const double cell_us = 1e-6 * (wide ? (cached ? 30.0 : 42.0) : (cached ? 18.0 : 21.6));
   // Non-temporal stores leave the L2 to the halo lines: FP32 rows of whole 64-byte
   // blocks whose buffers pass the cache gain (MLUPS without and with: 128^3 32.6k,
