@@ -65,6 +65,7 @@ struct culbm_ctx {
   bool dump_pending = false;
   // pinned ring of the large copies to the host (copy_out), made by the first one
   char* stage = nullptr;
+  bool stage_due = false;  // a copy that the ring would have served has been made
   hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // per-launch timing (culbm_profile_steps): an event pair around every launch
   bool prof = false;
@@ -753,7 +754,10 @@ struct HostCopy {
 // (and fault its pages in) while the next ones arrive.  The four fields, before
 // and after: 96x96x90 (13 MB) 2.0 -> 0.85 ms, 288x272x280 (351 MB) 35 -> 9.4 ms,
 // 384^3 (906 MB) 88 -> 21.6 ms.  Below 8 MB starting the threads costs as much.
-constexpr size_t kStageChunk = size_t(4) << 20, kStageLeast = size_t(8) << 20;
+// Making the ring takes 1.5 to 1.9 ms, which one copy below kStageOnce does not
+// win back, so there a context's second copy makes it.  Chunks of 1 or 2 MB copy
+// 351 MB in 19.3 or 12.7 ms.
+constexpr size_t kStageChunk = size_t(4) << 20, kStageLeast = size_t(8) << 20, kStageOnce = size_t(24) << 20;
 constexpr int kStages = 4, kCopyThreads = 8;
 
 // Threads that copy the parts of a chunk; they live for one copy_out.
@@ -867,7 +871,9 @@ int copy_out_staged(culbm_ctx* ctx, const std::vector<HostCopy>& copies) {
 int copy_out(culbm_ctx* ctx, const std::vector<HostCopy>& copies) {
   size_t total = 0;
   for (const HostCopy& c : copies) total += c.bytes;
-  if (total >= kStageLeast && stage_ready(ctx)) {
+  const bool staged = total >= kStageOnce || (total >= kStageLeast && ctx->stage_due);
+  ctx->stage_due |= total >= kStageLeast;
+  if (staged && stage_ready(ctx)) {
     try {
       return copy_out_staged(ctx, copies);
     } catch (const std::exception&) {

@@ -26,8 +26,9 @@ def filled(dim, seed=0):
                                  (1048577, 1, 1), (257, 131, 127)])
 def test_fields_arrive_unchanged(dim):
     lat, fields = filled(dim)
-    for got, want in zip(lat.macros(), fields):
-        assert np.array_equal(got, want)
+    for _ in range(2):  # the ring serves the smaller ones from the second copy on
+        for got, want in zip(lat.macros(), fields):
+            assert np.array_equal(got, want)
     one = np.empty(lat.shape, np.float32)
     _lib.check(_lib.lib().culbm_get_macros(lat._ctx, None, None, _lib.ptr(one), None), lat._ctx)
     assert np.array_equal(one, fields[2])
