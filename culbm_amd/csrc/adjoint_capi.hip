@@ -279,6 +279,7 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
   const size_t state = size_t(27) * size_t(n) * sizeof(typename S::T);
   const size_t mu_b = size_t(27) * size_t(n) * 4;
   const uint32_t obj_blk = uint32_t(std::max<size_t>((obj_idx.size() + kBlock - 1) / kBlock, 1));
+  const uint32_t obj_waves = uint32_t((obj_idx.size() + 63) / 64);
   const size_t fixed = 2 * mu_b + size_t(n) * 4 + size_t(4 * n_equ) * 8 +
                        size_t(27 * n_keep) * 4 + size_t(a.nblk) * 8 + size_t(obj_blk) * 8 +
                        obj_idx.size() * 12 + 2 * state + size_t(n) * 4 + 20 * 256;
@@ -319,7 +320,7 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
   int rc = CULBM_OK;
   for (auto& s : slot) mem.plan(&s, state, sizeof(typename S::T));
   for (auto& w : work) mem.plan(&w, state, sizeof(typename S::T));
-  for (auto& m : mu) mem.plan(&m, mu_b, 4);
+  for (auto& m : mu) mem.plan(&m, mu_b, 8);  // FP64: mu[0] holds J's sums until it is needed
   mem.plan(&d_aux, size_t(n) * 4, 4);
   mem.plan(&d_wobj, size_t(n) * 4, 4);
   if (sp.want_f0) mem.plan(&d_carry, size_t(27 * n_keep) * 4, 4);
@@ -392,15 +393,18 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
     o.w = d_w;
     o.count = uint32_t(obj_idx.size());
     o.mu = m;
-    o.j_acc = m ? nullptr : d_j;
-    hipLaunchKernelGGL((k_objective<S>), dim3(obj_blk), dim3(kBlock), 0, ctx->stream, o);
+    o.j_wave = m ? nullptr : reinterpret_cast<double*>(mu[0]);
+    const uint32_t block = objective_block(o.count);
+    hipLaunchKernelGGL((k_objective<S>), dim3((o.count + block - 1) / block), dim3(block), 0, ctx->stream, o);
     ++launches;
   };
   // a work buffer that is not `busy`
   auto free_work = [&](const void* busy) { return work[0] != busy ? work[0] : work[1]; };
 
   AdjTimer timer{ctx, sp.timing != 0, {}};
-  // ---- first sweep: J, the sweep checkpoints, f^N
+  // ---- first sweep: J (its sums in mu[0], at most 8 bytes of 108 a cell), the
+  // sweep checkpoints, f^N
+  if ((rc = zero_device(ctx, mu[0], size_t(obj_waves) * 8))) return rc;
   if ((rc = timer.enter(0))) return rc;
   const void* cur = slot[0];
   size_t next_store = 0;
@@ -419,6 +423,9 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
     t += n;
   }
   if ((rc = timer.close())) return rc;
+  if (obj_waves)
+    hipLaunchKernelGGL(k_objective_sum, dim3((obj_waves + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream,
+                       reinterpret_cast<const double*>(mu[0]), obj_waves, d_j);
   HIPCHK(ctx, hipGetLastError());
   // the context moves on to f^N
   hipLaunchKernelGGL((k_pull_to_plain<S>), dim3(a.nblk), dim3(kBlock), 0, ctx->stream, a, cur, mu[1]);
