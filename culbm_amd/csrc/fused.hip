@@ -15,18 +15,19 @@
 // only.
 //
 // What bounds it, at 288x272x280 with 60 spheres on 96x8 tiles: FP32 the bytes,
-// 131 per update counted (77 read of an ideal 54, 54 written) at 5.4 TB/s, above
-// the 5.25 TB/s the population pattern streams at; 16-bit the VALU (77 % busy)
-// and the bytes (77 per update) together.  A ring of all three planes in LDS (54
-// values per A cell, 32x16 FP32 tiles, EQU inputs loaded on demand, every
-// direction base held in scalar registers that spilled to vector lanes) ran 35.3k
-// MLUPS in FP32, 53.4k in FP16, 45.3k with stochastic rounding; this march 42.6k,
-// 62.5k and 54.3k.  Of that, FP32: the wide tile and its waits +20 %; FP16: the
-// same +4 %, computing in units of the storage scale +8 %, one barrier per plane
-// +6 %.  Measured and left out: gathers two planes ahead (fewer waves or spills:
-// FP32 64x8 34.5k), two workgroups of 32x12 per CU (29.5k), releasing the LDS
-// before the second step's arithmetic (spills, 35.8k), non-temporal loads (30.3k;
-// of the rows no other tile reads only, equal).
+// 128 per update counted (74 read of an ideal 54, 54 written) at 5.5 TB/s, above
+// the 5.25 TB/s the population pattern streams at; 16-bit the VALU, 90 % busy
+// (97 % with stochastic rounding; 76 and 71 bytes per update).  A ring of all
+// three planes in LDS (54 values per A cell, 32x16 FP32 tiles, EQU inputs loaded
+// on demand, every direction base held in scalar registers that spilled to vector
+// lanes) ran 35.3k MLUPS in FP32, 53.4k in FP16, 45.3k with stochastic rounding;
+// this march 42.6k, 62.5k and 54.3k (FP32 43.2k with non-temporal stores).  Of
+// that, FP32: the wide tile and its waits +20 %; FP16: the same +4 %, computing in
+// units of the storage scale +8 %, one barrier per plane +6 %.  Measured and left
+// out: gathers two planes ahead (fewer waves or spills: FP32 64x8 34.5k), two
+// workgroups of 32x12 per CU (29.5k), releasing the LDS before the second step's
+// arithmetic (spills, 35.8k), non-temporal loads (30.3k; of the rows no other
+// tile reads only, equal).
 //
 // The intermediate is kept in the storage format, exactly as a plain
 // step would have stored it, so two fused steps equal two plain steps bit for
