@@ -150,9 +150,14 @@ bool adj_check_plan(const AdjPlan& p) {
   return next == -1;
 }
 
-// Device workspace of one culbm_adjoint call, released on every exit path: one
-// allocation that the arrays share.  An allocation each (38 of them at 128^3,
-// every 20 steps) took 2.2 ms to make and 10 ms to give back, a tenth of the call.
+// Device workspace of one culbm_adjoint call: one allocation that the arrays
+// share.  An allocation each (38 of them at 128^3, every 20 steps) took 2.2 ms to
+// make and 10 ms to give back, a tenth of the call.  Up to kAdjKeep bytes stay
+// with the context for its next call (an optimisation loop makes many) and are
+// freed with it: where the process had just given back gigabytes, the allocation
+// of 727 MB took 7 ms and more of a call that takes 5.3 with it kept.
+constexpr int64_t kAdjKeep = int64_t(1) << 30;
+
 struct AdjBuffers {
   culbm_ctx* ctx;
   void* base = nullptr;
@@ -161,7 +166,12 @@ struct AdjBuffers {
   explicit AdjBuffers(culbm_ctx* c) : ctx(c) {}
   ~AdjBuffers() {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (base) (void)hipFree(base);
+    if (base && base != ctx->adj_ws) (void)hipFree(base);
+  }
+  void drop_kept() {
+    if (ctx->adj_ws) (void)hipFree(ctx->adj_ws);
+    ctx->adj_ws = nullptr;
+    ctx->adj_ws_bytes = 0;
   }
   // packed at the elements' own alignment: the cap counts the arrays' sizes
   template <class T>
@@ -171,10 +181,19 @@ struct AdjBuffers {
     bytes += int64_t(std::max<size_t>(nbytes, 256));
   }
   int make() {
-    if (hipMalloc(&base, size_t(bytes)) != hipSuccess) {
-      base = nullptr;
-      (void)hipGetLastError();
-      return fail(ctx, CULBM_ERR_HIP, "adjoint workspace: hipMalloc of %zu bytes failed", size_t(bytes));
+    if (bytes <= ctx->adj_ws_bytes) {
+      base = ctx->adj_ws;
+    } else {
+      drop_kept();
+      if (hipMalloc(&base, size_t(bytes)) != hipSuccess) {
+        base = nullptr;
+        (void)hipGetLastError();
+        return fail(ctx, CULBM_ERR_HIP, "adjoint workspace: hipMalloc of %zu bytes failed", size_t(bytes));
+      }
+      if (bytes <= kAdjKeep) {
+        ctx->adj_ws = base;
+        ctx->adj_ws_bytes = bytes;
+      }
     }
     for (const auto& p : parts) *p.first = static_cast<char*>(base) + p.second;
     return CULBM_OK;
@@ -287,7 +306,7 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
   if (cap == 0) {
     size_t fr = 0, tot = 0;
     HIPCHK(ctx, hipMemGetInfo(&fr, &tot));
-    cap = int64_t(double(fr) * 0.9);
+    cap = int64_t(double(fr + size_t(ctx->adj_ws_bytes)) * 0.9);
   }
   int32_t slots;
   if (sp.checkpoint_every > 0) {

@@ -67,6 +67,9 @@ struct culbm_ctx {
   char* stage = nullptr;
   bool stage_due = false;  // a copy that the ring would have served has been made
   hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  // workspace of the last culbm_adjoint, kept for the next one where it is small
+  void* adj_ws = nullptr;
+  int64_t adj_ws_bytes = 0;
   // per-launch timing (culbm_profile_steps): an event pair around every launch
   bool prof = false;
   size_t prof_used = 0;
@@ -1223,6 +1226,7 @@ int culbm_destroy(culbm_ctx* ctx) {
   for (hipGraphExec_t g : ctx->pass_graph)
     if (g) (void)hipGraphExecDestroy(g);
   for (hipEvent_t e : ctx->prof_ev) (void)hipEventDestroy(e);
+  if (ctx->adj_ws) (void)hipFree(ctx->adj_ws);
   for (hipEvent_t e : ctx->stage_ev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
