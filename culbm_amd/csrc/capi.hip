@@ -1479,7 +1479,7 @@ int culbm_get_info(culbm_ctx* ctx, culbm_info* info) {
   if (!info) return fail(ctx, CULBM_ERR_INVALID, "info is NULL");
   std::memset(info, 0, sizeof(*info));
   info->step = ctx->step;
-  info->device_bytes = ctx->device_bytes;
+  info->device_bytes = ctx->device_bytes + ctx->adj_ws_bytes;
   const bool pairs = fused_pairs(ctx);
   info->wave_depth = blocked(ctx->cfg) && (pairs || ctx->cfg.opt_policy == CULBM_OPT_MIXED) ? ctx->fused.zchunk : ctx->wave_depth;
   info->bytes_per_pop = ctx->bpp;

@@ -98,7 +98,8 @@ typedef struct culbm_config {
 
 typedef struct culbm_info {
   int64_t step;               /* cumulative steps taken                      */
-  int64_t device_bytes;       /* bytes of device memory held                 */
+  int64_t device_bytes;       /* bytes of device memory held, the workspace
+                               * kept by culbm_adjoint included              */
   int32_t wave_depth;         /* chunk depth in use (blocked policies)       */
   int32_t launches_per_pass;  /* kernel launches per pass of inner_loop steps */
   int32_t bytes_per_pop;      /* 4 (FP32) or 2 (FP16/BF16)                   */
@@ -243,7 +244,8 @@ typedef struct culbm_adjoint_stats {
  * objective's w).  grad_rho/ux/uy/uz: nx*ny*nz doubles each or NULL, zero
  * outside EQU cells.  grad_f0: 27*nx*ny*nz floats ([27][nz][ny][nx]) or NULL;
  * required when spec->want_f0.  Fails with CULBM_ERR_INVALID when the
- * checkpoints do not fit mem_cap. */
+ * checkpoints do not fit mem_cap.  A workspace of up to 1 GiB stays with the
+ * context for its next call. */
 int culbm_adjoint(culbm_ctx* ctx, const culbm_adjoint_spec* spec, const double* weight,
                   culbm_adjoint_stats* stats, double* grad_rho, double* grad_ux,
                   double* grad_uy, double* grad_uz, float* grad_f0);
