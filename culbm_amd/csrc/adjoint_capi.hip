@@ -163,7 +163,8 @@ struct AdjBuffers {
   void* base = nullptr;
   std::vector<std::pair<void**, size_t>> parts;  // where each array's address goes, and its offset
   int64_t bytes = 0;
-  explicit AdjBuffers(culbm_ctx* c) : ctx(c) {}
+  int64_t cap;  // of the call's spec (0: none): a kept workspace above it is given back
+  AdjBuffers(culbm_ctx* c, int64_t mem_cap) : ctx(c), cap(mem_cap) {}
   ~AdjBuffers() {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (base && base != ctx->adj_ws) (void)hipFree(base);
@@ -181,7 +182,7 @@ struct AdjBuffers {
     bytes += int64_t(std::max<size_t>(nbytes, 256));
   }
   int make() {
-    if (bytes <= ctx->adj_ws_bytes) {
+    if (bytes <= ctx->adj_ws_bytes && (cap == 0 || ctx->adj_ws_bytes <= cap)) {
       base = ctx->adj_ws;
     } else {
       drop_kept();
@@ -329,7 +330,7 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
   const AdjPlan plan = adj_make_plan(N, sp.checkpoint_every, slots);
   if (!adj_check_plan(plan)) return fail(ctx, CULBM_ERR_STATE, "inconsistent checkpoint schedule");
 
-  AdjBuffers mem(ctx);
+  AdjBuffers mem(ctx, sp.mem_cap);
   std::vector<void*> slot(size_t(plan.slots), nullptr);
   void* work[2] = {nullptr, nullptr};
   float* mu[2] = {nullptr, nullptr};

@@ -219,7 +219,8 @@ typedef struct culbm_adjoint_spec {
   int32_t t_begin, t_end;    /* objective window, 0 <= t_begin <= t_end <= N          */
   int32_t checkpoint_every;  /* k > 0: keep f^0, f^k, f^2k, ...; 0: binomial schedule */
   int32_t want_f0;           /* also return dJ/df^0                                    */
-  int64_t mem_cap;           /* device bytes the call may allocate; 0: 90% of free     */
+  int64_t mem_cap;           /* device bytes the workspace may take, one kept from an
+                              * earlier call included; 0: 90% of free memory           */
   int32_t timing;            /* fill the ms_* fields (device events per phase)         */
   int32_t max_slots;         /* binomial: at most this many states held (0: no limit)  */
   int32_t reserved[4];
@@ -229,7 +230,7 @@ typedef struct culbm_adjoint_stats {
   double objective;          /* J                                                      */
   double grad_inv_tau;       /* dJ/dinvTau                                             */
   int64_t forward_steps;     /* forward steps run, the first sweep included            */
-  int64_t device_bytes;      /* workspace allocated by the call                        */
+  int64_t device_bytes;      /* workspace the call uses                                */
   int32_t slots;             /* states held as checkpoints                             */
   int32_t launches;          /* kernel launches                                        */
   float ms_sweep;            /* first forward sweep (with the objective)               */

@@ -16,3 +16,20 @@ def test_device_bytes_counts_the_kept_workspace():
     lat.close()
     assert fake.fake_bytes() == 0
     """)
+
+
+def test_memory_cap_bounds_a_workspace_kept_from_an_earlier_call():
+    fakehip.run("""
+    lat = Lattice(LatticeConfig(domain=(24, 20, 16)))
+    w = np.ones(lat.shape)
+    base = fake.fake_bytes()
+    lat.adjoint(w, 40, (1, 40), checkpoint_every=1)
+    cap = (fake.fake_bytes() - base) // 4
+    assert lat.adjoint(w, 40, (1, 40), mem_cap=cap).stats["device_bytes"] <= cap
+    assert fake.fake_bytes() - base <= cap
+    held = fake.fake_bytes()  # a later call without a cap, or one that fits, takes what is there
+    lat.adjoint(w, 2, (1, 2))
+    lat.adjoint(w, 40, (1, 40), mem_cap=cap)
+    assert fake.fake_bytes() == held
+    lat.close()
+    """)
