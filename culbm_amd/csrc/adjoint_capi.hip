@@ -153,26 +153,20 @@ bool adj_check_plan(const AdjPlan& p) {
 // Device workspace of one culbm_adjoint call: one allocation that the arrays
 // share.  An allocation each (38 of them at 128^3, every 20 steps) took 2.2 ms to
 // make and 10 ms to give back, a tenth of the call.  Up to kAdjKeep bytes stay
-// with the context for its next call (an optimisation loop makes many) and are
-// freed with it: where the process had just given back gigabytes, the allocation
-// of 727 MB took 7 ms and more of a call that takes 5.3 with it kept.
-constexpr int64_t kAdjKeep = int64_t(1) << 30;
-
+// with the context for its next call (an optimisation loop makes many): where the
+// process had just given back gigabytes, the allocation of 727 MB took 7 ms and
+// more of a call that takes 5.3 with it kept.
 struct AdjBuffers {
   culbm_ctx* ctx;
   void* base = nullptr;
+  int64_t base_bytes = 0;
   std::vector<std::pair<void**, size_t>> parts;  // where each array's address goes, and its offset
   int64_t bytes = 0;
   int64_t cap;  // of the call's spec (0: none): a kept workspace above it is given back
   AdjBuffers(culbm_ctx* c, int64_t mem_cap) : ctx(c), cap(mem_cap) {}
   ~AdjBuffers() {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (base && base != ctx->adj_ws) (void)hipFree(base);
-  }
-  void drop_kept() {
-    if (ctx->adj_ws) (void)hipFree(ctx->adj_ws);
-    ctx->adj_ws = nullptr;
-    ctx->adj_ws_bytes = 0;
+    if (base) keep(ctx, base, base_bytes);
   }
   // packed at the elements' own alignment: the cap counts the arrays' sizes
   template <class T>
@@ -182,19 +176,15 @@ struct AdjBuffers {
     bytes += int64_t(std::max<size_t>(nbytes, 256));
   }
   int make() {
-    if (bytes <= ctx->adj_ws_bytes && (cap == 0 || ctx->adj_ws_bytes <= cap)) {
-      base = ctx->adj_ws;
-    } else {
-      drop_kept();
-      if (hipMalloc(&base, size_t(bytes)) != hipSuccess) {
+    base = take_kept(ctx, &base_bytes);
+    if (base_bytes < bytes || (cap > 0 && base_bytes > cap)) {
+      if (base) (void)hipFree(base);
+      base = nullptr;
+      if (device_malloc(ctx->cfg.device, &base, size_t(bytes)) != hipSuccess) {
         base = nullptr;
-        (void)hipGetLastError();
         return fail(ctx, CULBM_ERR_HIP, "adjoint workspace: hipMalloc of %zu bytes failed", size_t(bytes));
       }
-      if (bytes <= kAdjKeep) {
-        ctx->adj_ws = base;
-        ctx->adj_ws_bytes = bytes;
-      }
+      base_bytes = bytes;
     }
     for (const auto& p : parts) *p.first = static_cast<char*>(base) + p.second;
     return CULBM_OK;
@@ -306,8 +296,9 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
   int64_t cap = sp.mem_cap;
   if (cap == 0) {
     size_t fr = 0, tot = 0;
+    std::lock_guard<std::mutex> lock(g_kept_mu);  // what is kept is there for the taking
     HIPCHK(ctx, hipMemGetInfo(&fr, &tot));
-    cap = int64_t(double(fr + size_t(ctx->adj_ws_bytes)) * 0.9);
+    cap = int64_t(double(int64_t(fr) + kept_bytes(c.device)) * 0.9);
   }
   int32_t slots;
   if (sp.checkpoint_every > 0) {

@@ -67,9 +67,11 @@ struct culbm_ctx {
   char* stage = nullptr;
   bool stage_due = false;  // a copy that the ring would have served has been made
   hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
-  // workspace of the last culbm_adjoint, kept for the next one where it is small
+  // workspace of the last culbm_adjoint, kept for the next one where it is small,
+  // and the next context that keeps one (both under g_kept_mu)
   void* adj_ws = nullptr;
   int64_t adj_ws_bytes = 0;
+  culbm_ctx* kept_next = nullptr;
   // per-launch timing (culbm_profile_steps): an event pair around every launch
   bool prof = false;
   size_t prof_used = 0;
@@ -912,8 +914,94 @@ int zero_device(culbm_ctx* ctx, void* p, size_t bytes) {
 
 size_t ddf_bytes(const culbm_ctx* ctx) { return size_t(27) * size_t(ctx->dstride) * size_t(ctx->bpp); }
 
+// ---- workspaces kept between culbm_adjoint calls ---------------------------------
+// A block is listed only while no call uses it (its stream has been waited for),
+// so any thread may free it: a context that keeps one makes room by freeing the
+// others' oldest beyond kAdjKeep bytes on the device, and an allocation that
+// fails frees them all and is made again.
+constexpr int64_t kAdjKeep = int64_t(1) << 30;
+std::mutex g_kept_mu;
+culbm_ctx* g_kept = nullptr;  // oldest first
+
+// The caller holds g_kept_mu and owns the block afterwards.
+void* unlist_kept(culbm_ctx* ctx, int64_t* bytes) {
+  for (culbm_ctx** q = &g_kept; *q; q = &(*q)->kept_next)
+    if (*q == ctx) {
+      *q = ctx->kept_next;
+      break;
+    }
+  void* p = ctx->adj_ws;
+  *bytes = ctx->adj_ws_bytes;
+  ctx->adj_ws = nullptr;
+  ctx->adj_ws_bytes = 0;
+  ctx->kept_next = nullptr;
+  return p;
+}
+
+int64_t kept_bytes(int32_t device) {  // the caller holds g_kept_mu
+  int64_t sum = 0;
+  for (const culbm_ctx* q = g_kept; q; q = q->kept_next)
+    if (q->cfg.device == device) sum += q->adj_ws_bytes;
+  return sum;
+}
+
+// Frees kept workspaces of the device, oldest first, until at most `bytes` stay.
+bool trim_kept(int32_t device, int64_t bytes) {  // the caller holds g_kept_mu
+  bool freed = false;
+  for (culbm_ctx* q = g_kept; q && kept_bytes(device) > bytes;) {
+    culbm_ctx* next = q->kept_next;
+    if (q->cfg.device == device) {
+      int64_t b;
+      (void)hipFree(unlist_kept(q, &b));
+      freed = true;
+    }
+    q = next;
+  }
+  return freed;
+}
+
+void* take_kept(culbm_ctx* ctx, int64_t* bytes) {
+  std::lock_guard<std::mutex> lock(g_kept_mu);
+  return unlist_kept(ctx, bytes);
+}
+
+// Keeps an idle block with the context (which holds none), or frees it.
+void keep(culbm_ctx* ctx, void* p, int64_t bytes) {
+  if (bytes > kAdjKeep) {
+    (void)hipFree(p);
+    return;
+  }
+  std::lock_guard<std::mutex> lock(g_kept_mu);
+  trim_kept(ctx->cfg.device, kAdjKeep - bytes);
+  culbm_ctx** q = &g_kept;
+  while (*q) q = &(*q)->kept_next;
+  *q = ctx;
+  ctx->adj_ws = p;
+  ctx->adj_ws_bytes = bytes;
+}
+
+// hipMalloc on the current device, `device`; a failure leaves no error behind for
+// the check after a later launch.
+hipError_t device_malloc(int32_t device, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> lock(g_kept_mu);
+    if (!trim_kept(device, 0)) return e;
+  }
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+template <class T>
+hipError_t device_malloc(int32_t device, T** p, size_t bytes) {
+  return device_malloc(device, reinterpret_cast<void**>(p), bytes);
+}
+
 int alloc(culbm_ctx* ctx, void** p, size_t bytes) {
-  HIPCHK(ctx, hipMalloc(p, bytes));
+  HIPCHK(ctx, device_malloc(ctx->cfg.device, p, bytes));
   ctx->device_bytes += int64_t(bytes);
   return CULBM_OK;
 }
@@ -1226,7 +1314,8 @@ int culbm_destroy(culbm_ctx* ctx) {
   for (hipGraphExec_t g : ctx->pass_graph)
     if (g) (void)hipGraphExecDestroy(g);
   for (hipEvent_t e : ctx->prof_ev) (void)hipEventDestroy(e);
-  if (ctx->adj_ws) (void)hipFree(ctx->adj_ws);
+  int64_t kept = 0;
+  if (void* p = take_kept(ctx, &kept)) (void)hipFree(p);
   for (hipEvent_t e : ctx->stage_ev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
@@ -1300,7 +1389,7 @@ int culbm_init_ddf(culbm_ctx* ctx, int32_t mode) {
   ctx->parity = 1;
   if (mode == CULBM_INIT_FEQ) {
     float* plain = nullptr;
-    HIPCHK(ctx, hipMalloc(&plain, size_t(27) * size_t(ctx->n) * 4));
+    HIPCHK(ctx, device_malloc(ctx->cfg.device, &plain, size_t(27) * size_t(ctx->n) * 4));
     StepArgs a = full_args(ctx);
     hipLaunchKernelGGL(k_feq_plain, dim3(a.nblk), dim3(kBlock), 0, ctx->stream, a, plain);
     int rc = CULBM_OK;
@@ -1409,7 +1498,7 @@ int culbm_get_ddf(culbm_ctx* ctx, float* ddf) {
   HIPCHK(ctx, hipSetDevice(ctx->cfg.device));
   const size_t bytes = size_t(27) * size_t(ctx->n) * 4;
   float* plain = nullptr;
-  HIPCHK(ctx, hipMalloc(&plain, bytes));
+  HIPCHK(ctx, device_malloc(ctx->cfg.device, &plain, bytes));
   int rc = by_storage(ctx->cfg.storage, [&](auto s) { return download_plain<decltype(s)>(ctx, plain); });
   if (!rc) rc = copy_out(ctx, {{ddf, plain, bytes}});
   (void)hipStreamSynchronize(ctx->stream);
@@ -1431,7 +1520,7 @@ int culbm_set_ddf(culbm_ctx* ctx, const float* ddf) {
     set_scale(ctx, derived_scale(ctx->cfg.storage, std::max(ctx->state_bound, double(m))));
   }
   float* plain = nullptr;
-  HIPCHK(ctx, hipMalloc(&plain, bytes));
+  HIPCHK(ctx, device_malloc(ctx->cfg.device, &plain, bytes));
   int rc = CULBM_OK;
   if (hipMemcpyAsync(plain, ddf, bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
     rc = fail(ctx, CULBM_ERR_HIP, "host-to-device copy failed");
@@ -1450,7 +1539,7 @@ int culbm_moment_sums(culbm_ctx* ctx, uint32_t flag_mask, double* sums) {
   if (!sums) return fail(ctx, CULBM_ERR_INVALID, "sums is NULL");
   HIPCHK(ctx, hipSetDevice(ctx->cfg.device));
   double* work = nullptr;
-  HIPCHK(ctx, hipMalloc(&work, moment_sums_work_bytes()));
+  HIPCHK(ctx, device_malloc(ctx->cfg.device, &work, moment_sums_work_bytes()));
   int rc = moment_sums_launch(ctx, flag_mask, work);
   if (!rc && hipMemcpyAsync(sums, work + 4 * kSumParts, 4 * sizeof(double), hipMemcpyDeviceToHost,
                             ctx->stream) != hipSuccess)
@@ -1479,7 +1568,10 @@ int culbm_get_info(culbm_ctx* ctx, culbm_info* info) {
   if (!info) return fail(ctx, CULBM_ERR_INVALID, "info is NULL");
   std::memset(info, 0, sizeof(*info));
   info->step = ctx->step;
-  info->device_bytes = ctx->device_bytes + ctx->adj_ws_bytes;
+  {
+    std::lock_guard<std::mutex> lock(g_kept_mu);
+    info->device_bytes = ctx->device_bytes + ctx->adj_ws_bytes;
+  }
   const bool pairs = fused_pairs(ctx);
   info->wave_depth = blocked(ctx->cfg) && (pairs || ctx->cfg.opt_policy == CULBM_OPT_MIXED) ? ctx->fused.zchunk : ctx->wave_depth;
   info->bytes_per_pop = ctx->bpp;
@@ -1533,8 +1625,8 @@ int culbm_probe_cells(int32_t device, int32_t op, float inv_tau, float* f, const
   float *df = nullptr, *din = nullptr, *dout = nullptr;
   int rc = CULBM_OK;
   const size_t fb = size_t(n) * 27 * 4, qb = size_t(n) * 4 * 4;
-  if (hipMalloc(&df, fb) != hipSuccess || hipMalloc(&din, qb) != hipSuccess ||
-      hipMalloc(&dout, qb) != hipSuccess)
+  if (device_malloc(device, &df, fb) != hipSuccess || device_malloc(device, &din, qb) != hipSuccess ||
+      device_malloc(device, &dout, qb) != hipSuccess)
     rc = fail(nullptr, CULBM_ERR_HIP, "allocation failed");
   if (!rc && op != 1 && hipMemcpy(df, f, fb, hipMemcpyHostToDevice) != hipSuccess)
     rc = fail(nullptr, CULBM_ERR_HIP, "copy failed");
@@ -1564,8 +1656,8 @@ int culbm_probe_codec(int32_t device, int32_t storage, float scale, const float*
   float *din = nullptr, *ddec = nullptr;
   uint16_t* denc = nullptr;
   int rc = CULBM_OK;
-  if (hipMalloc(&din, size_t(n) * 4) != hipSuccess || hipMalloc(&ddec, size_t(n) * 4) != hipSuccess ||
-      hipMalloc(&denc, size_t(n) * 2) != hipSuccess)
+  if (device_malloc(device, &din, size_t(n) * 4) != hipSuccess || device_malloc(device, &ddec, size_t(n) * 4) != hipSuccess ||
+      device_malloc(device, &denc, size_t(n) * 2) != hipSuccess)
     rc = fail(nullptr, CULBM_ERR_HIP, "allocation failed");
   if (!rc && hipMemcpy(din, in, size_t(n) * 4, hipMemcpyHostToDevice) != hipSuccess)
     rc = fail(nullptr, CULBM_ERR_HIP, "copy failed");
@@ -1625,8 +1717,8 @@ int culbm_probe_bandwidth(int32_t device, int32_t mode, int64_t bytes, int32_t i
     if (e != hipSuccess && !rc) rc = fail(nullptr, CULBM_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
     return rc == CULBM_OK;
   };
-  if (hipMalloc(&a, n4 * 16 + 256) != hipSuccess || hipMalloc(&b, n4 * 16 + 256) != hipSuccess ||
-      hipMalloc(&bad, 256) != hipSuccess)
+  if (device_malloc(device, &a, n4 * 16 + 256) != hipSuccess || device_malloc(device, &b, n4 * 16 + 256) != hipSuccess ||
+      device_malloc(device, &bad, 256) != hipSuccess)
     rc = fail(nullptr, CULBM_ERR_HIP, "allocation failed");
   if (!rc && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess))
     rc = fail(nullptr, CULBM_ERR_HIP, "event creation failed");

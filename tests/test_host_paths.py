@@ -33,3 +33,45 @@ def test_memory_cap_bounds_a_workspace_kept_from_an_earlier_call():
     assert fake.fake_bytes() == held
     lat.close()
     """)
+
+
+def test_kept_workspaces_are_bounded_per_device_and_given_back():
+    fakehip.run("""
+    GiB = 1 << 30
+
+    def made(dim, steps):
+        lat = Lattice(LatticeConfig(domain=dim))
+        lat.adjoint(np.ones(lat.shape), steps, (1, steps), checkpoint_every=1)
+        return lat
+
+    lats = [made((64, 60, 50), 18) for _ in range(4)]  # about 0.44 GB of workspace each
+    own = [lat.info()["device_bytes"] for lat in lats]
+    assert sum(own) == fake.fake_bytes()
+    base = min(own)
+    kept = [b - base for b in own]
+    assert kept[:2] == [0, 0] and min(kept[2:]) > 0.4e9 and sum(kept) <= GiB, kept
+    # an allocation that only fits once they are given back, by a context that keeps
+    # none, by one that does and by a new one
+    plain = 27 * 4 * 64 * 60 * 50
+    for call in (lats[0].get_ddf, lambda: lats[1].set_ddf(np.zeros((27, 50, 60, 64), np.float32)),
+                 lambda: lats[0].init_ddf("feq"), lats[0].moment_sums,
+                 lambda: Lattice(LatticeConfig(domain=(16, 16, 16))).close()):
+        fake.fake_limit(1 << 40)
+        lats[3].adjoint(np.ones(lats[3].shape), 18, (1, 18), checkpoint_every=1)
+        assert lats[3].info()["device_bytes"] > base
+        fake.fake_limit(fake.fake_bytes())
+        call()
+        assert lats[3].info()["device_bytes"] == base
+    # one that never fits still fails, and the context goes on
+    fake.fake_limit(fake.fake_bytes() + plain // 2)
+    try:
+        lats[0].get_ddf()
+        raise SystemExit("no error")
+    except _lib.CulbmError as e:
+        assert e.code == _lib.ERR_HIP
+    fake.fake_limit(1 << 40)
+    lats[0].get_ddf()
+    for lat in lats:
+        lat.close()
+    assert fake.fake_bytes() == 0
+    """)
