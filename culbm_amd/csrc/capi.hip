@@ -1006,6 +1006,11 @@ int alloc(culbm_ctx* ctx, void** p, size_t bytes) {
   return CULBM_OK;
 }
 
+// Bytes of populations (as allocated) and flags up to which the Infinity Cache
+// (256 MB) serves one step what the step before it wrote: the middle of a range in
+// which sizes run two ways.
+constexpr double kCacheHolds = 237e6;
+
 // Planes per wavefront chunk.  FP32 in place and pull: a launch-size target
 // (1.4M cells in place, 1.25M pull) capped by the cache-fitting depth (D + T + 1
 // planes within ~160 MB of the 256 MB Infinity Cache) or half the domain,
@@ -1017,8 +1022,7 @@ int alloc(culbm_ctx* ctx, void** p, size_t bytes) {
 // nears the cache; at 256^3 and 384^3 the optimum moved by a plane or two from
 // run to run, within +-4 %); FP16 pull 46.7k at 16 planes, 44.5k at 32.  FP16
 // in place peaked at 172-190 MB in every run: 256^3 46.2k at 33 planes, 42.2k
-// at 40; 384^3 47.7k at 12, 44.7k at 18; 288x272x280 44.9-48.2k at 32-34.  At
-// 128^3 the cache-fitting 83 planes beat one whole-domain chunk by 16 % (FP32).
+// at 40; 384^3 47.7k at 12, 44.7k at 18; 288x272x280 44.9-48.2k at 32-34.
 int32_t auto_depth(const culbm_ctx* ctx) {
   const double cells = double(ctx->cfg.nx) * ctx->cfg.ny;
   const int32_t T = std::max(1, ctx->cfg.inner_loop);
@@ -1029,11 +1033,13 @@ int32_t auto_depth(const culbm_ctx* ctx) {
     const int32_t d = std::max(fit, int32_t(std::ceil(1.6e6 / cells)));
     return std::max(2, std::min(d, nz));
   }
-  // FP32 in place: a domain the cache holds is one launch a step (MLUPS against
-  // the chunk rule's two launches: 128x128x90 28.4k vs 27.0k, 157x93x141 25.1k vs
-  // 24.3k, 100x100x200 27.4k vs 26.7k; 128^3, 226 MB, ran 23.4k or 28.9k and
-  // keeps its chunks, 27.5k; 192x160x176 22.4k vs 25.1k)
-  if (ctx->inplace && 27.0 * ctx->bpp * cells * nz <= 224e6) return nz;
+  // FP32 in place: a domain that the cache holds is one launch a step.  Against the
+  // chunk rule's two launches, 8 contexts a size: 31 sizes from 125 to 236 MB +2 to
+  // +10 % (128^3, 234 MB, 28.1k vs 27.5k MLUPS; 157x93x141, 233 MB, 25.4k vs
+  // 24.4k; 200x104x100, 232 MB, 28.7k vs 27.6k) but 136x128x120 and 123x127x130
+  // -1 to +3 % and 101x140x133 -5 to -12 %; of 13 sizes from 237 to 266 MB, 10
+  // -6 to -18 % (128x128x132, 241 MB, 23.7k vs 26.5k), 3 below 240 MB +2 to +4 %.
+  if (ctx->inplace && 27.0 * ctx->bpp * double(ctx->dstride) + cells * nz <= kCacheHolds) return nz;
   const double plane = cells * (27.0 * ctx->bpp * (ctx->inplace ? 1 : 2) + 1.0);
   const double budget = 160.0 * 1024 * 1024;
   const int32_t fit = std::max(int32_t(budget / plane) - T - 1, 2);
