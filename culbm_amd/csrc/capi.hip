@@ -1008,7 +1008,9 @@ int alloc(culbm_ctx* ctx, void** p, size_t bytes) {
 
 // Bytes of populations (as allocated) and flags up to which the Infinity Cache
 // (256 MB) serves one step what the step before it wrote: the middle of a range in
-// which sizes run two ways.
+// which sizes run two ways.  In place see auto_depth; plain pull steps run 49k to
+// 55k MLUPS in 16 bits up to 200 MB, 44k to 55k from there to 250 MB and 43k to 45k
+// at 257 MB, in FP32 29k at 224 MB, 25k to 28k at 237 to 253 MB, 23k at 283 MB.
 constexpr double kCacheHolds = 237e6;
 
 // Planes per wavefront chunk.  FP32 in place and pull: a launch-size target
@@ -1073,12 +1075,20 @@ int32_t auto_depth(const culbm_ctx* ctx) {
 // 203x170x119 102x7 (34.9k; 96x8 27.4k), at 48x200x150 48x17 (34.7k; 64x13
 // 33.6k); FP16 at 33x270x280 33x27 (51.9k; 64x13 34.3k).
 //
-// A plain step costs 3.3 us and a rate that steps down once its two buffers
-// pass the cache.  Measured either side of the line, two steps per launch
-// against plain steps: FP32 at 80^3 25.6k vs 28.0k MLUPS, at 96^3 36.5k vs
-// 28.7k; FP16 at 107x109x78 48.3k vs 50.6k, at 150x220x90 50.5k vs 44.5k; FP16
-// with stochastic rounding at 203x170x119 43.2k vs 45.0k, at 192x160x176 49.0k
-// vs 46.0k.
+// A plain step costs 3.3 us and a rate that falls where its two buffers pass the
+// cache: at once on some shapes, late on others (FP16 62x181x186, 228 MB, 44k MLUPS,
+// 144x118x118, 219 MB, 54k), so the cost ramps from one to the other.  Where the
+// cache holds them the model puts pairs too high (by 5 to 35 % in FP32, 5 to 20 %
+// in 16 bits) and they are taken up to 1.09 times the plain steps' time; beyond it
+// ties go to the plain steps, and BF16's pairs, 4 % slower than FP16's, need 8 %.
+// Of 366 chosen and drawn sizes from 40 to 590 MB none takes pairs and loses 3 %, 41
+// keep plain steps that pairs would beat by 3 to 29 % (narrow ones most).
+// Two steps per launch against plain steps in MLUPS: FP32 at 84x84x44 25.1k vs
+// 26.2k, at 80^3 30.5k vs 27.8k, at 64x100x100 32.0k vs 27.6k; FP16 at 107x109x78
+// 49.9k vs 50.0k, at 267x61x91 51.7k vs 54.0k, at 120^3 55.5k vs 52.9k, at 128^3
+// 56.4k vs 53.1k; BF16 at 257x57x155 51.3k vs 53.6k, at 144^2x136 52.0k vs 45.4k;
+// FP16 with stochastic rounding at 203x170x119 43.4k vs 44.6k, at 192x160x144
+// 46.9k vs 44.4k.
 FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   const culbm_config& c = ctx->cfg;
   const bool wide = ctx->bpp == 4;
@@ -1090,7 +1100,7 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   // once more, and per row of A cells: fixed, per line read
   const double write = 128e-6 * (wide ? 0.37 : (ctx->sr ? 0.669 : 0.544));
   const double edge = wide ? 0.38 : (ctx->sr ? 0.08 : 0.11);
-  const double row = 128e-6 * (wide ? 0.0 : (ctx->sr ? 0.020 : 0.037)), line = 128e-6 * (wide ? 0.03 : 0.0);
+  const double row = 128e-6 * (wide ? 0.0 : (ctx->sr ? 0.020 : 0.037)), row_line = 128e-6 * (wide ? 0.03 : 0.0);
   const bool given = c.opt_policy == CULBM_OPT_MIXED && c.wave_depth > 0;
   FusedPlan best;
   double best_us = 0.0;
@@ -1110,7 +1120,7 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
       const double plane_us = fix + wa * std::ceil((tx + 2) * (p.ty + 2) / 256.0) + wb * std::ceil(tx * p.ty / 256.0);
       const bool aligned = tx * ctx->bpp % 64 == 0 && c.nx * ctx->bpp % 64 == 0;
       const double out = double(p.tiles_x) * c.ny * c.nz * (tx * ctx->bpp / 128.0 + (aligned ? 0.0 : edge));
-      const double reads = tiles * (p.ty + 2) * (row + line * ((tx + 2) * ctx->bpp / 128.0 + 1.0));
+      const double reads = tiles * (p.ty + 2) * (row + row_line * ((tx + 2) * ctx->bpp / 128.0 + 1.0));
       for (int n = 1; n <= (given ? 1 : std::min(64, c.nz)); ++n) {
         p.zchunk = given ? std::min(c.wave_depth, c.nz) : int32_t((int64_t(c.nz) + n - 1) / n);
         p.nchunk = int32_t((int64_t(c.nz) + p.zchunk - 1) / p.zchunk);
@@ -1124,18 +1134,19 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
       }
     }
   }
-  // (at 226 MB, FP16 128^3, plain steps ran 46k or 54k MLUPS from one context to
-  // the next and the pairs 53k to 55k; with stochastic rounding 45k or 52k, and 45k)
-  const bool cached = 2.0 * 27.0 * ctx->bpp * cells < (ctx->sr ? 240e6 : 210e6);
-  const double cell_us = 1e-6 * (wide ? (cached ? 30.0 : 42.0) : (cached ? 18.0 : 21.6));
+  const double held = (2.0 * 27.0 * ctx->bpp + 1.0) * cells / kCacheHolds;
+  const double past = std::min(std::max((held - 0.84) / 0.32, 0.0), 1.0);
+  const double cell_us = 1e-6 * (wide ? 30.0 + 12.0 * past : 18.0 + 3.6 * past);
   // Non-temporal stores leave the L2 to the halo lines: FP32 rows of whole 64-byte
   // blocks whose buffers pass the cache gain (MLUPS without and with: 128^3 32.6k,
   // 34.1k; 192x160x176 38.9k, 39.7k; 256^3 37.6k, 40.3k; 288x272x280 42.6k, 43.2k);
   // blocks shared by two tiles are then written twice (203x170x119 34.9k, 25.3k),
   // cached buffers miss (96^3 36.6k, 34.0k), and 16-bit rows go either way.
-  best.nt = wide && !cached && c.nx % 16 == 0 && best.tx % 16 == 0;
-  // a launch's own start and fill count where it is short; ties go to the plain steps
-  best.pays = best_us + (wide ? 2.0 : 6.0) < (ctx->sr ? 1.0 : (c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95)) * 2.0 * (3.3 + cells * cell_us);
+  best.nt = wide && 216.0 * cells >= 210e6 && c.nx % 16 == 0 && best.tx % 16 == 0;
+  const double far_line = c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95;
+  const double line = ctx->sr ? 1.0 : 1.09 + (far_line - 1.09) * past;
+  // a launch's own start and fill count where it is short
+  best.pays = best_us + (wide ? 2.0 : 6.0) < line * 2.0 * (3.3 + cells * cell_us);
   return best;
 }
 

@@ -27,3 +27,23 @@ def test_in_place_one_launch_a_step_follows_the_allocated_bytes():
         lat.close()
     assert 4 < one < 20
     """)
+
+
+def test_pull_steps_in_pairs_where_they_measured_faster():
+    """Sizes on either side of the line, plain pull steps with no depth given; the
+    cache's share does not depend on the rounding mode."""
+    fakehip.run("""
+    pairs = [("fp32", "nearest", (80, 80, 80)), ("fp32", "nearest", (101, 99, 97)), ("fp32", "nearest", (40, 104, 262)),
+             ("fp16", "nearest", (120, 120, 120)), ("fp16", "nearest", (128, 128, 128)), ("fp16", "nearest", (62, 181, 186)),
+             ("bf16", "nearest", (144, 128, 120)), ("fp16", "stochastic", (192, 160, 144))]
+    plain = [("fp32", "nearest", (72, 72, 72)), ("fp32", "nearest", (84, 84, 44)), ("fp32", "nearest", (64, 64, 64)),
+             ("fp16", "nearest", (107, 109, 78)), ("fp16", "nearest", (267, 61, 91)), ("bf16", "nearest", (257, 57, 155)),
+             ("fp16", "stochastic", (130, 126, 126)), ("fp16", "stochastic", (203, 170, 119))]
+    for want, rows in (("k_fused2", pairs), ("k_pull", plain)):
+        for storage, rounding, dim in rows:
+            lat = Lattice(LatticeConfig(domain=dim, storage=storage, rounding=rounding))
+            fake.fake_clear()
+            lat.step(2)
+            assert set(launched()) == {want}, (storage, rounding, dim, launched())
+            lat.close()
+    """)
