@@ -1137,12 +1137,14 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   const double held = (2.0 * 27.0 * ctx->bpp + 1.0) * cells / kCacheHolds;
   const double past = std::min(std::max((held - 0.84) / 0.32, 0.0), 1.0);
   const double cell_us = 1e-6 * (wide ? 30.0 + 12.0 * past : 18.0 + 3.6 * past);
-  // Non-temporal stores leave the L2 to the halo lines: FP32 rows of whole 64-byte
-  // blocks whose buffers pass the cache gain (MLUPS without and with: 128^3 32.6k,
-  // 34.1k; 192x160x176 38.9k, 39.7k; 256^3 37.6k, 40.3k; 288x272x280 42.6k, 43.2k);
+  // Non-temporal stores leave the L2 to the halo lines and miss the cache: FP32
+  // rows of whole 64-byte blocks gain once the cache holds little of the two
+  // buffers (MLUPS without and with: 96x104x112, 242 MB, 38.6k, 36.5k; 128x112x96,
+  // 297 MB, 35.1k, 34.3k; 112^3, 303 MB, equal; 128x112x112, 347 MB, 33.1k, 34.8k;
+  // 192x160x176 38.9k, 39.7k; 256^3 37.6k, 40.3k; 288x272x280 42.6k, 43.2k);
   // blocks shared by two tiles are then written twice (203x170x119 34.9k, 25.3k),
-  // cached buffers miss (96^3 36.6k, 34.0k), and 16-bit rows go either way.
-  best.nt = wide && 216.0 * cells >= 210e6 && c.nx % 16 == 0 && best.tx % 16 == 0;
+  // and 16-bit rows go either way.
+  best.nt = wide && held > 1.3 && c.nx % 16 == 0 && best.tx % 16 == 0;
   const double far_line = c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95;
   const double line = ctx->sr ? 1.0 : 1.09 + (far_line - 1.09) * past;
   // a launch's own start and fill count where it is short

@@ -47,3 +47,18 @@ def test_pull_steps_in_pairs_where_they_measured_faster():
             assert set(launched()) == {want}, (storage, rounding, dim, launched())
             lat.close()
     """)
+
+
+def test_non_temporal_stores_only_beyond_the_cache():
+    """FP32 rows of whole 64-byte blocks: the stores pass the cache by only where it
+    holds little of the two buffers."""
+    fakehip.run("""
+    for dim, nt in [((96, 96, 96), 0), ((112, 96, 96), 0), ((96, 104, 112), 0), ((128, 112, 112), 1), ((160, 136, 136), 1),
+                    ((127, 127, 127), 0)]:
+        lat = Lattice(LatticeConfig(domain=dim))
+        fake.fake_clear()
+        lat.step(2)
+        (name,) = fake.fake_log().decode().split()
+        assert "StoreF32ELb0ELb%dE" % nt in name, (dim, name)
+        lat.close()
+    """)
