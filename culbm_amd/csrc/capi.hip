@@ -463,28 +463,24 @@ int launch_step(culbm_ctx* ctx, StepArgs a, int32_t z0, int32_t z1, int parity, 
 // by the same chunk one launch earlier, and no (plane, step) is computed twice.
 // A chunk's working set (D + T planes) is sized for the Infinity Cache.  The
 // schedule is exported (culbm_wave_schedule) for the host-side hazard check.
+//
+// A chunk as deep as the domain would leave the skewed ends to a second chunk,
+// T - 1 launches of a few planes each, so there every step is one launch over all
+// planes.  32^3 in place, I = 5: 9 launches a pass and 213 us for 20 steps, against
+// 5 and 129 us; 157x93x141 FP16 950 us against 867 us.
 template <class F>
-int for_each_wave_launch(int32_t nz, int32_t D, int32_t T, F&& f) {
-  const int32_t K = (nz + T - 1 + D - 1) / D;
-  for (int32_t k = 0; k < K; ++k) {
+int for_each_wave_launch(int32_t nz, int32_t depth, int32_t T, F&& f) {
+  const int64_t D = depth < nz ? depth : int64_t(nz) + T - 1;
+  const int64_t K = (int64_t(nz) + T - 1 + D - 1) / D;
+  for (int64_t k = 0; k < K; ++k) {
     for (int32_t t = 1; t <= T; ++t) {
-      const int32_t lo = std::max(0, k * D - (t - 1));
-      const int32_t hi = std::min(nz, (k + 1) * D - (t - 1));
+      const int32_t lo = int32_t(std::max<int64_t>(0, k * D - (t - 1)));
+      const int32_t hi = int32_t(std::min<int64_t>(nz, (k + 1) * D - (t - 1)));
       if (lo >= hi) continue;
       if (int rc = f(lo, hi, t)) return rc;
     }
   }
   return CULBM_OK;
-}
-
-// Chunk depth of a pass of T steps.  A chunk as deep as the domain leaves the
-// skewed ends to a second chunk, T - 1 launches of a few planes each; T - 1
-// planes more make every step one launch.  32^3 in place, I = 5: 9 launches a
-// pass and 213 us for 20 steps, against 5 and 129 us; 157x93x141 FP16 950 us
-// against 867 us.
-int32_t pass_depth(const culbm_ctx* ctx, int32_t T) {
-  const int32_t nz = ctx->cfg.nz;
-  return ctx->wave_depth < nz || nz > INT32_MAX - T ? ctx->wave_depth : nz + T - 1;
 }
 
 template <class S>
@@ -493,7 +489,7 @@ int wave_pass(culbm_ctx* ctx, int32_t T) {
   const uint32_t base = uint32_t(ctx->step);
   // a pending dump rides on the first step: its launches cover every plane once
   const bool dump = ctx->dump_pending;
-  const int rc = for_each_wave_launch(ctx->cfg.nz, pass_depth(ctx, T), T, [&](int32_t lo, int32_t hi, int32_t t) {
+  const int rc = for_each_wave_launch(ctx->cfg.nz, ctx->wave_depth, T, [&](int32_t lo, int32_t hi, int32_t t) {
     if (!ctx->inplace) {
       a.src = ctx->buf[(ctx->cur + t - 1) & 1];
       a.dst = ctx->buf[(ctx->cur + t) & 1];
@@ -1604,7 +1600,7 @@ int culbm_get_info(culbm_ctx* ctx, culbm_info* info) {
     info->launches_per_pass = c.inner_loop;
   } else {
     int32_t cnt = 0;
-    for_each_wave_launch(c.nz, pass_depth(ctx, c.inner_loop), c.inner_loop, [&](int32_t, int32_t, int32_t) {
+    for_each_wave_launch(c.nz, ctx->wave_depth, c.inner_loop, [&](int32_t, int32_t, int32_t) {
       ++cnt;
       return CULBM_OK;
     });

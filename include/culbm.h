@@ -279,8 +279,9 @@ int culbm_blocking_axis(int32_t dom, int32_t blk, int32_t iter, int32_t* num, in
 
 /* Launch schedule of one temporal-blocking pass of the dynamic and static
  * policies (the z-wavefront that replaces the reference's per-tile launch loop,
- * simulator_expt_platform.cu:749-872): for a domain of nz planes, chunks of
- * `depth` planes and `steps` steps, launches[3k..3k+2] = (z0, z1, t) of the
+ * simulator_expt_platform.cu:749-872; pull contexts that take their steps in
+ * pairs run none): for a domain of nz planes, chunks of `depth` planes (nz or
+ * more: every step one launch) and `steps` steps, launches[3k..3k+2] = (z0, z1, t) of the
  * k-th launch in issue order, step t (1-based) over planes [z0, z1).
  * launches may be NULL to count only.  Host only (the hazard checker's input). */
 int culbm_wave_schedule(int32_t nz, int32_t depth, int32_t steps, int32_t* launches, int32_t max_launches,

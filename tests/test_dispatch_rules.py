@@ -62,3 +62,28 @@ def test_non_temporal_stores_only_beyond_the_cache():
         assert "StoreF32ELb0ELb%dE" % nt in name, (dim, name)
         lat.close()
     """)
+
+
+def test_the_exported_schedule_is_the_one_that_runs():
+    """Launches of a pass against culbm_wave_schedule at the depth the context
+    reports: chunked, as deep as the domain and beyond, chosen and given."""
+    fakehip.run("""
+    from culbm_amd.blocking import wave_schedule
+    for dim, storage in (((24, 20, 16), "fp32"), ((24, 20, 16), "fp16"), ((96, 90, 80), "fp32"), ((192, 160, 176), "fp32"),
+                         ((192, 160, 176), "fp16"), ((5, 4, 1), "fp32")):
+        for sp, op in ((1, 1), (1, 3), (0, 1), (0, 3)):
+            for depth in (0, 3, dim[2] - 1, dim[2], dim[2] + 7):
+                if sp == 0 and depth == 0:
+                    continue  # pull steps left to the library may run in pairs
+                for loop in (1, 5):
+                    lat = Lattice(LatticeConfig(domain=dim, storage=storage, stream_policy=sp, opt_policy=op,
+                                                inner_loop=loop, wave_depth=depth, block_dim=(1, 1, 1), grid_dim=dim))
+                    want = wave_schedule(dim[2], lat.info()["wave_depth"], loop)
+                    fake.fake_clear()
+                    lat.step(loop)
+                    what = (dim, storage, sp, op, depth, loop, lat.info())
+                    grids = [fake.fake_grid(k) for k in range(len(want) + 1)]
+                    assert grids == [-(-(z1 - z0) * dim[0] * dim[1] // 256) for z0, z1, t in want] + [-1], what
+                    assert lat.info()["launches_per_pass"] == len(want), what
+                    lat.close()
+    """)
