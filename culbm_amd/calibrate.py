@@ -24,8 +24,10 @@ is set by where a chunk's working set meets the Infinity Cache, by launch
 ramp-up and tail and by the workgroup order, which no closed form captured
 across sizes.  So the selector measures: it times the dynamic policy over
 candidate depths (launches of 0.6M to 3.2M cells, plus the automatic choice)
-and innerLoop values on this GPU and domain, and reports the fastest
-(--waveDepth / --innerLoop of the CLI):
+and innerLoop values on this GPU and domain, and reports the fastest: its
+requested_depth and inner_loop are the --waveDepth and --innerLoop of the CLI
+(depth 0 leaves it to the library, which takes pull steps in pairs where that is
+faster; such a row says "pairs" and has no wave_depth):
 
     python -m culbm_amd.calibrate --select --domain 288 272 280 [--storage fp16]
         [--stream 1] [--inner-loop 5 6] [--init-state DIR]
@@ -77,7 +79,8 @@ def select(domain: Tuple[int, int, int], stream_policy: int = 1, storage: str = 
            develop: int = 1000) -> dict:
     """Time the dynamic policy (optPolicy 3) over candidate depths and innerLoop
     values; return every candidate's MLUPS (best of three timed runs) and the
-    fastest.  `state` defaults to the seeded obstacle channel of `domain`.
+    fastest.  A candidate is run again by passing its requested_depth as the
+    depth; wave_depth is the wavefront's chunk, 0 where steps ran in pairs.  `state` defaults to the seeded obstacle channel of `domain`.
     Each candidate first runs `develop` untimed steps from rest: the step rate
     depends on the population values (a flow at rest, whose shifted
     populations are zero, runs up to 7 % faster than the developed flow)."""
@@ -102,7 +105,8 @@ def select(domain: Tuple[int, int, int], stream_policy: int = 1, storage: str = 
             lat.step(develop + 2 * il)
             k = steps or il * max(2, math.ceil(4e8 / (n * il)))
             ms = min(lat.time_steps(k) for _ in range(3))
-            return n * k / (ms * 1e-3) / 1e6, lat.info()["wave_depth"]
+            pairs = lat.profile_steps(2)["launches"] == 1
+            return n * k / (ms * 1e-3) / 1e6, 0 if pairs else lat.info()["wave_depth"], pairs
         finally:
             lat.close()
 
@@ -110,8 +114,9 @@ def select(domain: Tuple[int, int, int], stream_policy: int = 1, storage: str = 
     rows = []
     for il in inner_loops:
         for d in cands:
-            mlups, used = timed(il, d)
-            rows.append({"inner_loop": il, "requested_depth": d, "wave_depth": used, "mlups": round(mlups, 1)})
+            mlups, used, pairs = timed(il, d)
+            rows.append({"inner_loop": il, "requested_depth": d, "wave_depth": used, "pairs": pairs,
+                         "mlups": round(mlups, 1)})
     best = max(rows, key=lambda r: r["mlups"])
     return {"domain": list(domain), "stream_policy": stream_policy, "storage": storage, "rounding": rounding,
             "best": best, "candidates": rows}

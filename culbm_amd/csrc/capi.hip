@@ -1588,7 +1588,7 @@ int culbm_get_info(culbm_ctx* ctx, culbm_info* info) {
     info->device_bytes = ctx->device_bytes + ctx->adj_ws_bytes;
   }
   const bool pairs = fused_pairs(ctx);
-  info->wave_depth = blocked(ctx->cfg) && (pairs || ctx->cfg.opt_policy == CULBM_OPT_MIXED) ? ctx->fused.zchunk : ctx->wave_depth;
+  info->wave_depth = ctx->cfg.opt_policy == CULBM_OPT_MIXED ? ctx->fused.zchunk : ctx->wave_depth;
   info->bytes_per_pop = ctx->bpp;
   info->storage_scale = ctx->scale;
   const culbm_config& c = ctx->cfg;

@@ -91,7 +91,9 @@ typedef struct culbm_config {
   int32_t device;           /* --devId                                       */
   int32_t storage;          /* CULBM_STORAGE_*                               */
   float storage_scale;      /* 16-bit scale (power of two); 0 = per run      */
-  int32_t wave_depth;       /* planes per wavefront chunk; 0 = automatic     */
+  int32_t wave_depth;       /* planes per chunk of the wavefront, or of the mixed
+                             * policy's pairs of steps; 0 = automatic, and pull
+                             * then takes pairs or not, whichever is faster   */
   int32_t rounding;         /* CULBM_ROUND_* of the 16-bit stores            */
   int32_t reserved[6];
 } culbm_config;
@@ -100,7 +102,12 @@ typedef struct culbm_info {
   int64_t step;               /* cumulative steps taken                      */
   int64_t device_bytes;       /* bytes of device memory held, the workspace
                                * kept by culbm_adjoint included              */
-  int32_t wave_depth;         /* chunk depth in use (blocked policies)       */
+  int32_t wave_depth;         /* blocked policies: planes per chunk of the wavefront
+                               * (mixed: of the two-step kernel), as a given
+                               * wave_depth would set them.  A pull context without
+                               * a given one takes its steps in pairs where that is
+                               * faster and runs no wavefront then:
+                               * launches_per_pass is (inner_loop + 1) / 2    */
   int32_t launches_per_pass;  /* kernel launches per pass of inner_loop steps */
   int32_t bytes_per_pop;      /* 4 (FP32) or 2 (FP16/BF16)                   */
   float storage_scale;        /* scale in use                                */
@@ -129,8 +136,8 @@ int culbm_set_state(culbm_ctx* ctx, const uint32_t* flag, const float* rho, cons
  * the step counter. */
 int culbm_init_ddf(culbm_ctx* ctx, int32_t mode);
 
-/* Advance exactly nsteps steps (any policy; blocked policies run passes of
- * inner_loop steps and a shorter final pass). */
+/* Advance exactly nsteps steps.  The wavefront runs passes of inner_loop steps and
+ * a shorter final pass; pull contexts may take steps two at a time (same bits). */
 int culbm_step(culbm_ctx* ctx, int32_t nsteps);
 
 /* One window of the reference's run(): time the step launches of `dstep`

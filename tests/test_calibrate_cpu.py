@@ -32,3 +32,27 @@ def test_select_rejects_an_empty_candidate_list():
         select((16, 16, 16), depths=())
     with pytest.raises(ValueError):
         select((16, 16, 16), inner_loops=())
+
+
+def test_selector_does_not_report_a_depth_that_did_not_run():
+    """Pull left to the library takes pairs at this size: no wavefront depth is
+    reported for it, and a context's info names the depth that an explicit setting
+    would take, not the two-step kernel's."""
+    import fakehip
+
+    fakehip.run("""
+    from culbm_amd.calibrate import select
+    dim = (112, 104, 96)
+    rows = select(dim, stream_policy=0, depths=(0, 24), steps=4, develop=2)["candidates"]
+    assert [(r["requested_depth"], r["wave_depth"], r["pairs"]) for r in rows] == [(0, 0, True), (24, 24, False)], rows
+    rows = select(dim, stream_policy=1, depths=(0, 24), steps=4, develop=2)["candidates"]
+    assert [(r["wave_depth"], r["pairs"]) for r in rows] == [(96, False), (24, False)], rows
+    for op in (1, 3):
+        lat = Lattice(LatticeConfig(domain=dim, opt_policy=op))
+        assert lat.info()["launches_per_pass"] == 3
+        auto = lat.info()["wave_depth"]
+        lat.close()
+        lat = Lattice(LatticeConfig(domain=dim, opt_policy=op, wave_depth=auto))
+        assert lat.info()["wave_depth"] == auto == 60
+        lat.close()
+    """)
