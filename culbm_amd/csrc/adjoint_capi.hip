@@ -550,8 +550,10 @@ int culbm_adjoint(culbm_ctx* ctx, const culbm_adjoint_spec* spec, const double* 
   HIPCHK(ctx, hipSetDevice(ctx->cfg.device));
   if (int rc = flush_dump(ctx)) return rc;
   double* g[4] = {grad_rho, grad_ux, grad_uy, grad_uz};
-  return by_storage(ctx->cfg.storage, [&](auto st) {
-    return adjoint_impl<decltype(st)>(ctx, s, weight, stats, g, s.want_f0 ? grad_f0 : nullptr);
+  return no_throw(ctx, [&] {
+    return by_storage(ctx->cfg.storage, [&](auto st) {
+      return adjoint_impl<decltype(st)>(ctx, s, weight, stats, g, s.want_f0 ? grad_f0 : nullptr);
+    });
   });
 }
 
@@ -559,11 +561,13 @@ int culbm_adjoint_plan(int32_t nsteps, int32_t checkpoint_every, int32_t slots,
                        int64_t* forward_steps, int32_t* slots_used) {
   if (nsteps < 1 || checkpoint_every < 0 || (checkpoint_every == 0 && slots < 1))
     return fail(nullptr, CULBM_ERR_INVALID, "plan needs nsteps >= 1 and every > 0 or slots >= 1");
-  const AdjPlan p = adj_make_plan(nsteps, checkpoint_every, slots);
-  if (!adj_check_plan(p)) return fail(nullptr, CULBM_ERR_STATE, "inconsistent checkpoint schedule");
-  if (forward_steps) *forward_steps = p.forward;
-  if (slots_used) *slots_used = p.slots;
-  return CULBM_OK;
+  return no_throw(nullptr, [&]() -> int {
+    const AdjPlan p = adj_make_plan(nsteps, checkpoint_every, slots);
+    if (!adj_check_plan(p)) return fail(nullptr, CULBM_ERR_STATE, "inconsistent checkpoint schedule");
+    if (forward_steps) *forward_steps = p.forward;
+    if (slots_used) *slots_used = p.slots;
+    return CULBM_OK;
+  });
 }
 
 }  // extern "C"

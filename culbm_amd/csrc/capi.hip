@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -88,11 +89,22 @@ int fail(culbm_ctx* ctx, int code, const char* fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
-  if (ctx)
-    ctx->err = buf;
-  else
-    g_create_err = buf;
+  try {
+    (ctx ? ctx->err : g_create_err) = buf;
+  } catch (const std::exception&) {  // no memory for the message: the code alone
+  }
   return code;
+}
+
+// The entry points' own allocations on the host may fail, and nothing is thrown
+// across the C ABI.
+template <class F>
+int no_throw(culbm_ctx* ctx, F&& f) {
+  try {
+    return f();
+  } catch (const std::exception& e) {
+    return fail(ctx, CULBM_ERR_HIP, "host allocation failed: %s", e.what());
+  }
 }
 
 #define HIPCHK(ctx, expr)                                                                   \
@@ -836,14 +848,14 @@ bool stage_ready(culbm_ctx* ctx) {
   return true;
 }
 
-int copy_out_staged(culbm_ctx* ctx, const std::vector<HostCopy>& copies) {
+int copy_out_staged(culbm_ctx* ctx, const HostCopy* copies, int count) {
   ChunkCopiers pool;
   for (int k = 0; k < kCopyThreads; ++k) pool.threads.emplace_back(&ChunkCopiers::work, &pool, k);
   std::vector<ChunkCopiers::Job> chunks;  // src: device until it is posted
-  for (const HostCopy& c : copies)
-    for (size_t o = 0; o < c.bytes; o += kStageChunk)
-      chunks.push_back({static_cast<char*>(c.dst) + o, static_cast<const char*>(c.src) + o,
-                        std::min(kStageChunk, c.bytes - o)});
+  for (const HostCopy* c = copies; c != copies + count; ++c)
+    for (size_t o = 0; o < c->bytes; o += kStageChunk)
+      chunks.push_back({static_cast<char*>(c->dst) + o, static_cast<const char*>(c->src) + o,
+                        std::min(kStageChunk, c->bytes - o)});
   const int64_t n = int64_t(chunks.size());
   auto enqueue = [&](int64_t i) -> int {
     char* slot = ctx->stage + size_t(i % kStages) * kStageChunk;
@@ -869,21 +881,21 @@ int copy_out_staged(culbm_ctx* ctx, const std::vector<HostCopy>& copies) {
 }
 
 // Copies to pageable host memory; they are complete on return.
-int copy_out(culbm_ctx* ctx, const std::vector<HostCopy>& copies) {
+int copy_out(culbm_ctx* ctx, const HostCopy* copies, int count) {
   size_t total = 0;
-  for (const HostCopy& c : copies) total += c.bytes;
+  for (int k = 0; k < count; ++k) total += copies[k].bytes;
   const bool staged = total >= kStageOnce || (total >= kStageLeast && ctx->stage_due);
   ctx->stage_due |= total >= kStageLeast;
   if (staged && stage_ready(ctx)) {
     try {
-      return copy_out_staged(ctx, copies);
+      return copy_out_staged(ctx, copies, count);
     } catch (const std::exception&) {
       // no threads or memory to be had: the runtime's own copies, below
       (void)hipStreamSynchronize(ctx->stream);
     }
   }
-  for (const HostCopy& c : copies)
-    HIPCHK(ctx, hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, ctx->stream));
+  for (int k = 0; k < count; ++k)
+    HIPCHK(ctx, hipMemcpyAsync(copies[k].dst, copies[k].src, copies[k].bytes, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return CULBM_OK;
 }
@@ -1243,10 +1255,11 @@ int culbm_create(const culbm_config* cfg, culbm_ctx** out) {
   if (cfg->device >= ndev)
     return fail(nullptr, CULBM_ERR_INVALID, "devId %d out of range (%d devices)", cfg->device, ndev);
 
-  culbm_ctx* ctx = new culbm_ctx();
+  culbm_ctx* ctx = new (std::nothrow) culbm_ctx();
+  if (!ctx) return fail(nullptr, CULBM_ERR_HIP, "host allocation failed: context");
   ctx->cfg = *cfg;
   auto bail = [&](int rc) {
-    g_create_err = ctx->err;
+    g_create_err.swap(ctx->err);
     culbm_destroy(ctx);
     return rc;
   };
@@ -1307,12 +1320,12 @@ int culbm_create(const culbm_config* cfg, culbm_ctx** out) {
   }
 
   // reference defaults: all FLUID + DUMP, rho 1, u 0, rest populations
-  {
+  CK(no_throw(ctx, [&] {
     std::vector<uint32_t> fl(nb, CULBM_FLAG_LOAD | CULBM_FLAG_COLLIDE | CULBM_FLAG_STORE |
                                      CULBM_FLAG_DUMP_RHO | CULBM_FLAG_DUMP_VX |
                                      CULBM_FLAG_DUMP_VY | CULBM_FLAG_DUMP_VZ);
-    CK(culbm_set_state(ctx, fl.data(), nullptr, nullptr, nullptr, nullptr));
-  }
+    return culbm_set_state(ctx, fl.data(), nullptr, nullptr, nullptr, nullptr);
+  }));
   CK(culbm_init_ddf(ctx, CULBM_INIT_REST));
 #undef CK
 #undef HK
@@ -1378,7 +1391,14 @@ int culbm_set_state(culbm_ctx* ctx, const uint32_t* flag, const float* rho, cons
     if (src[k]) {
       HIPCHK(ctx, hipMemcpyAsync(dst[k], src[k], nb * 4, hipMemcpyHostToDevice, ctx->stream));
     } else {
-      if (fill.empty() || fill[0] != dflt[k]) fill.assign(nb, dflt[k]);
+      const int rc = no_throw(ctx, [&] {
+        if (fill.empty() || fill[0] != dflt[k]) fill.assign(nb, dflt[k]);
+        return int(CULBM_OK);
+      });
+      if (rc) {
+        (void)hipStreamSynchronize(ctx->stream);  // the caller's arrays may still be read
+        return rc;
+      }
       HIPCHK(ctx, hipMemcpyAsync(dst[k], fill.data(), nb * 4, hipMemcpyHostToDevice, ctx->stream));
       HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // `fill` is reused
     }
@@ -1450,7 +1470,7 @@ int culbm_profile_steps(culbm_ctx* ctx, int32_t nsteps, float* kernel_ms, int32_
   HIPCHK(ctx, hipSetDevice(ctx->cfg.device));
   ctx->prof = true;
   ctx->prof_used = 0;
-  const int rc = steps_dispatch(ctx, nsteps);
+  const int rc = no_throw(ctx, [&] { return steps_dispatch(ctx, nsteps); });
   ctx->prof = false;
   if (rc) return rc;
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1501,10 +1521,11 @@ int culbm_get_macros(culbm_ctx* ctx, float* rho, float* vx, float* vy, float* vz
   if (int rc = flush_dump(ctx)) return rc;
   float* dst[4] = {rho, vx, vy, vz};
   const float* src[4] = {ctx->rho, ctx->vx, ctx->vy, ctx->vz};
-  std::vector<HostCopy> copies;
+  HostCopy copies[4];
+  int count = 0;
   for (int k = 0; k < 4; ++k)
-    if (dst[k]) copies.push_back({dst[k], src[k], size_t(ctx->n) * 4});
-  return copy_out(ctx, copies);
+    if (dst[k]) copies[count++] = {dst[k], src[k], size_t(ctx->n) * 4};
+  return copy_out(ctx, copies, count);
 }
 
 int culbm_get_ddf(culbm_ctx* ctx, float* ddf) {
@@ -1515,7 +1536,8 @@ int culbm_get_ddf(culbm_ctx* ctx, float* ddf) {
   float* plain = nullptr;
   HIPCHK(ctx, device_malloc(ctx->cfg.device, &plain, bytes));
   int rc = by_storage(ctx->cfg.storage, [&](auto s) { return download_plain<decltype(s)>(ctx, plain); });
-  if (!rc) rc = copy_out(ctx, {{ddf, plain, bytes}});
+  const HostCopy copy{ddf, plain, bytes};
+  if (!rc) rc = copy_out(ctx, &copy, 1);
   (void)hipStreamSynchronize(ctx->stream);
   (void)hipFree(plain);
   return rc;

@@ -23,7 +23,6 @@ std::string g_log;  // names of the kernels launched, one a line
 std::vector<uint32_t> g_grids;
 long g_copies = 0, g_largest = 0;  // device-to-host copies
 int g_threads = 0;                 // most threads seen while one was waited for
-long g_new_left = -1;              // allocations until operator new fails (-1: never)
 char* g_known = nullptr;           // a range that hipPointerGetAttributes knows
 size_t g_known_bytes = 0;
 
@@ -33,13 +32,26 @@ struct Dim3 {
 
 }  // namespace
 
+extern "C" {
+long fake_new_left = -1;  // allocations until one fails (-1: none does); -1 again afterwards
+}
+
 void* operator new(size_t n) {
-  if (g_new_left >= 0 && g_new_left-- == 0) throw std::bad_alloc();
+  if (fake_new_left >= 0 && fake_new_left-- == 0) throw std::bad_alloc();
   if (void* p = std::malloc(n ? n : 1)) return p;
   throw std::bad_alloc();
 }
 void operator delete(void* p) noexcept { std::free(p); }
 void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+namespace {
+// The stand-in's own allocations never fail.
+struct Immune {
+  long left = fake_new_left;
+  Immune() { fake_new_left = -1; }
+  ~Immune() { fake_new_left = left; }
+};
+}  // namespace
 
 extern "C" {
 
@@ -51,7 +63,7 @@ long fake_grid(long k) { return k < long(g_grids.size()) ? long(g_grids[size_t(k
 long fake_copies() { return g_copies; }
 long fake_largest() { return g_largest; }
 int fake_threads() { return g_threads; }
-void fake_fail_new(long after) { g_new_left = after; }
+void fake_fail_new(long after) { fake_new_left = after; }
 void fake_known(void* p, size_t bytes) {
   g_known = static_cast<char*>(p);
   g_known_bytes = bytes;
@@ -74,6 +86,7 @@ void __hipRegisterFunction(void**, const void* host, char*, const char* name, un
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 int __hipPushCallConfiguration(Dim3 grid, Dim3, size_t, void*) {
+  Immune immune;
   g_grids.push_back(grid.x);
   return kOk;
 }
@@ -84,6 +97,7 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* shared, void** st
   return kOk;
 }
 int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void*) {
+  Immune immune;
   g_log += g_names.count(f) ? g_names[f] : std::string("?");
   g_log += '\n';
   return kOk;
@@ -94,6 +108,7 @@ int hipMalloc(void** p, size_t n) {
   if (g_bytes + n > g_limit) return kOutOfMemory;
   *p = std::calloc(n ? n : 1, 1);
   if (!*p) return kOutOfMemory;
+  Immune immune;
   g_held[*p] = n;
   g_bytes += n;
   return kOk;

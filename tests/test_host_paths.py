@@ -75,3 +75,60 @@ def test_kept_workspaces_are_bounded_per_device_and_given_back():
         lat.close()
     assert fake.fake_bytes() == 0
     """)
+
+
+def test_a_failing_host_allocation_never_throws_through_the_c_abi():
+    """operator new fails at its first, second, ... call within an entry point until
+    the entry point gets through: every outcome is a return code, and the context
+    works on."""
+    fakehip.run("""
+    lib = _lib.lib()
+
+    def outcomes(call):
+        codes = []
+        for k in range(500):
+            fake.fake_fail_new(k)
+            codes.append(call())
+            used_all = ctypes.c_long.in_dll(fake, "fake_new_left").value >= 0
+            fake.fake_fail_new(-1)
+            if used_all:
+                break
+        assert codes[-1] == _lib.OK and set(codes) <= {_lib.OK, _lib.ERR_HIP}, codes
+        return codes
+
+    big = Lattice(LatticeConfig(domain=(256, 128, 100)))  # 52 MB of fields: through the ring
+    small = Lattice(LatticeConfig(domain=(16, 12, 10)))
+    for lat in (small, big):
+        fields = [np.random.default_rng(k).random(lat.shape, dtype=np.float32) for k in range(4)]
+        lat.set_state(None, *fields)
+        out = [np.empty(lat.shape, np.float32) for _ in range(4)]
+        ptrs = [_lib.ptr(a) for a in out]
+        outcomes(lambda: lib.culbm_get_macros(lat._ctx, *ptrs))
+        assert all(np.array_equal(a, b) for a, b in zip(out, fields))
+    f = np.empty((27,) + small.shape, np.float32)
+    get_ddf, p = lib["culbm_get_ddf"], _lib.ptr(f)  # plain pointers: numpy's own conversions allocate too
+    outcomes(lambda: get_ddf(small._ctx, p))
+    p = _lib.ptr(fields[0])
+    outcomes(lambda: lib.culbm_set_state(small._ctx, None, None, p, None, None))
+    outcomes(lambda: lib.culbm_profile_steps(small._ctx, 3, None, None))
+    outcomes(lambda: lib.culbm_adjoint_plan(40, 0, 5, None, None))
+    w = np.ones(small.shape)
+    p = _lib.ptr(w)
+    spec, stats = _lib.AdjointSpec(), _lib.AdjointStats()
+    spec.nsteps, spec.t_begin, spec.t_end = 6, 1, 6
+    codes = outcomes(lambda: lib.culbm_adjoint(small._ctx, ctypes.byref(spec), p, ctypes.byref(stats),
+                                               None, None, None, None, None))
+    assert len(codes) > 5 and _lib.ERR_HIP in codes
+    cfg, held = LatticeConfig(domain=(16, 12, 10)).to_c(), fake.fake_bytes()
+
+    def create():
+        h = ctypes.c_void_p()
+        rc = lib.culbm_create(ctypes.byref(cfg), ctypes.byref(h))
+        assert (rc == _lib.OK) == bool(h.value)
+        if h.value:
+            lib.culbm_destroy(h)
+        assert fake.fake_bytes() == held
+        return rc
+
+    assert _lib.ERR_HIP in outcomes(create)
+    """)
