@@ -880,12 +880,23 @@ int copy_out_staged(culbm_ctx* ctx, const HostCopy* copies, int count) {
   return CULBM_OK;
 }
 
-// Copies to pageable host memory; they are complete on return.
+// Memory that the runtime knows (pinned, managed, on a device) takes a copy at the
+// link's rate as it is, and need not be the CPU's to write.
+bool pageable(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Copies to the caller's memory; they are complete on return.
 int copy_out(culbm_ctx* ctx, const HostCopy* copies, int count) {
   size_t total = 0;
   for (int k = 0; k < count; ++k) total += copies[k].bytes;
-  const bool staged = total >= kStageOnce || (total >= kStageLeast && ctx->stage_due);
+  bool staged = total >= kStageOnce || (total >= kStageLeast && ctx->stage_due);
   ctx->stage_due |= total >= kStageLeast;
+  for (int k = 0; k < count && staged; ++k)
+    staged = pageable(copies[k].dst) && pageable(static_cast<const char*>(copies[k].dst) + copies[k].bytes - 1);
   if (staged && stage_ready(ctx)) {
     try {
       return copy_out_staged(ctx, copies, count);

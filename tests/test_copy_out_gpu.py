@@ -60,3 +60,16 @@ def test_two_contexts_on_two_threads():
     assert not bad
     for lat, _ in made:
         lat.close()
+
+
+def test_into_pinned_memory():
+    torch = pytest.importorskip("torch")
+    lat, fields = filled((160, 150, 100), 5)
+    out = [torch.empty(lat.shape, dtype=torch.float32, pin_memory=True) for _ in range(4)]
+    for _ in range(2):
+        for t in out:
+            t.zero_()
+        _lib.check(_lib.lib().culbm_get_macros(lat._ctx, *[t.data_ptr() for t in out]), lat._ctx)
+        for t, want in zip(out, fields):
+            assert np.array_equal(t.numpy(), want)
+    lat.close()

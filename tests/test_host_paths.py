@@ -132,3 +132,33 @@ def test_a_failing_host_allocation_never_throws_through_the_c_abi():
 
     assert _lib.ERR_HIP in outcomes(create)
     """)
+
+
+def test_memory_that_the_runtime_knows_is_copied_to_directly():
+    """A caller's pinned (or managed, or device) array takes one copy a field; only
+    pageable memory goes through the ring's chunks."""
+    fakehip.run("""
+    lat = Lattice(LatticeConfig(domain=(256, 128, 100)))  # 13 MB a field
+    fields = [np.random.default_rng(k).random(lat.shape, dtype=np.float32) for k in range(4)]
+    lat.set_state(None, *fields)
+    block = np.empty((4,) + lat.shape, np.float32)
+    other = [np.empty(lat.shape, np.float32) for _ in range(4)]
+    fake.fake_known(block.ctypes.data, block.nbytes)
+    chunk, field = 4 << 20, fields[0].nbytes
+
+    def copy(out):
+        fake.fake_clear()
+        _lib.check(_lib.lib().culbm_get_macros(lat._ctx, *[_lib.ptr(a) for a in out]), lat._ctx)
+        assert all(np.array_equal(a, b) for a, b in zip(out, fields))
+        return fake.fake_copies(), fake.fake_largest()
+
+    for _ in range(2):
+        assert copy(other) == (16, chunk)
+        assert copy(list(block)) == (4, field)
+        assert copy(other[:3] + [block[3]]) == (4, field)
+    ddf = np.empty((27,) + lat.shape, np.float32)
+    fake.fake_known(ddf.ctypes.data, ddf.nbytes)
+    fake.fake_clear()
+    _lib.check(_lib.lib().culbm_get_ddf(lat._ctx, ddf), lat._ctx)
+    assert fake.fake_largest() == ddf.nbytes
+    """)
