@@ -1,6 +1,7 @@
 // Host side of the C ABI declared in include/culbm.h: context, buffers,
 // policy dispatch and the temporal-blocking wavefront schedule.
 #include <hip/hip_runtime.h>
+#include <sched.h>
 
 #include <algorithm>
 #include <cmath>
@@ -763,8 +764,9 @@ struct HostCopy {
 // A copy into pageable memory through the runtime fills the destination from
 // one thread: 10 GB/s into freshly mapped arrays, whose page faults that thread
 // takes too.  From kStageLeast bytes on, the copies go through a pinned ring of
-// kStages chunks at the link's rate and kCopyThreads threads move each chunk on
-// (and fault its pages in) while the next ones arrive.  The four fields, before
+// kStages chunks at the link's rate and up to kCopyThreads threads, one for each
+// CPU the process may use, move each chunk on (and fault its pages in) while the
+// next ones arrive.  The four fields, before
 // and after: 96x96x90 (13 MB) 2.0 -> 0.85 ms, 288x272x280 (351 MB) 35 -> 9.4 ms,
 // 384^3 (906 MB) 88 -> 21.6 ms.  Below 8 MB starting the threads costs as much.
 // Making the ring takes 1.5 to 1.9 ms, which one copy below kStageOnce does not
@@ -785,6 +787,7 @@ struct ChunkCopiers {
   Job job[kStages];
   int64_t posted = 0;            // chunks handed out
   int64_t done[kCopyThreads]{};  // chunks finished, per thread
+  int n = 0;                     // threads
   bool stop = false;
   std::vector<std::thread> threads;
 
@@ -797,10 +800,10 @@ struct ChunkCopiers {
         if (posted <= i) return;
         j = job[i % kStages];
       }
-      // whole pages per thread, so that no two fault the same one
-      const size_t part = (j.bytes / kCopyThreads + 4095) / 4096 * 4096;
+      // parts of a page's size, so that neighbours share at most one page
+      const size_t part = (j.bytes / size_t(n) + 4095) / 4096 * 4096;
       const size_t a = std::min(j.bytes, part * size_t(k));
-      const size_t b = k == kCopyThreads - 1 ? j.bytes : std::min(j.bytes, a + part);
+      const size_t b = k == n - 1 ? j.bytes : std::min(j.bytes, a + part);
       std::memcpy(j.dst + a, j.src + a, b - a);
       {
         std::lock_guard<std::mutex> lock(mu);
@@ -819,7 +822,7 @@ struct ChunkCopiers {
   }
   void wait(int64_t chunks) {  // until the first `chunks` chunks are copied
     std::unique_lock<std::mutex> lock(mu);
-    cv.wait(lock, [&] { return *std::min_element(done, done + kCopyThreads) >= chunks; });
+    cv.wait(lock, [&] { return *std::min_element(done, done + n) >= chunks; });
   }
   ~ChunkCopiers() {
     {
@@ -830,6 +833,12 @@ struct ChunkCopiers {
     for (std::thread& t : threads) t.join();
   }
 };
+
+int copy_threads() {
+  cpu_set_t set;
+  const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : kCopyThreads;
+  return std::min(std::max(cpus, 1), kCopyThreads);
+}
 
 bool stage_ready(culbm_ctx* ctx) {
   if (ctx->stage) return true;
@@ -850,7 +859,8 @@ bool stage_ready(culbm_ctx* ctx) {
 
 int copy_out_staged(culbm_ctx* ctx, const HostCopy* copies, int count) {
   ChunkCopiers pool;
-  for (int k = 0; k < kCopyThreads; ++k) pool.threads.emplace_back(&ChunkCopiers::work, &pool, k);
+  pool.n = copy_threads();
+  for (int k = 0; k < pool.n; ++k) pool.threads.emplace_back(&ChunkCopiers::work, &pool, k);
   std::vector<ChunkCopiers::Job> chunks;  // src: device until it is posted
   for (const HostCopy* c = copies; c != copies + count; ++c)
     for (size_t o = 0; o < c->bytes; o += kStageChunk)

@@ -162,3 +162,19 @@ def test_memory_that_the_runtime_knows_is_copied_to_directly():
     _lib.check(_lib.lib().culbm_get_ddf(lat._ctx, ddf), lat._ctx)
     assert fake.fake_largest() == ddf.nbytes
     """)
+
+
+def test_copying_threads_stay_within_the_cpus_the_process_may_use():
+    fakehip.run("""
+    import os
+    lat = Lattice(LatticeConfig(domain=(256, 128, 100)))
+    fields = [np.random.default_rng(k).random(lat.shape, dtype=np.float32) for k in range(4)]
+    lat.set_state(None, *fields)
+    cpus = sorted(os.sched_getaffinity(0))
+    for use in (1, min(3, len(cpus)), len(cpus)):
+        os.sched_setaffinity(0, set(cpus[:use]))
+        before = len(os.listdir("/proc/self/task"))
+        fake.fake_clear()
+        assert all(np.array_equal(a, b) for a, b in zip(lat.macros(), fields))
+        assert fake.fake_threads() - before == min(use, 8), (use, before, fake.fake_threads())
+    """)
