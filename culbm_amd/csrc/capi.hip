@@ -1147,7 +1147,7 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
       p.tiles_y = int32_t((int64_t(c.ny) + p.ty - 1) / p.ty);
       const double tiles = double(p.tiles_x) * p.tiles_y;
       const double plane_us = fix + wa * std::ceil((tx + 2) * (p.ty + 2) / 256.0) + wb * std::ceil(tx * p.ty / 256.0);
-      const bool aligned = tx * ctx->bpp % 64 == 0 && c.nx * ctx->bpp % 64 == 0;
+      const bool aligned = tx * ctx->bpp % 64 == 0 && c.nx % (64 / ctx->bpp) == 0;
       const double out = double(p.tiles_x) * c.ny * c.nz * (tx * ctx->bpp / 128.0 + (aligned ? 0.0 : edge));
       const double reads = tiles * (p.ty + 2) * (row + row_line * ((tx + 2) * ctx->bpp / 128.0 + 1.0));
       for (int n = 1; n <= (given ? 1 : std::min(64, c.nz)); ++n) {

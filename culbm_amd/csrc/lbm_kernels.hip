@@ -45,11 +45,12 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nblk) {
 // measured; 8 and 16 lead in every form).
 constexpr uint32_t kXcdGroup = 8;
 
-__device__ __forceinline__ uint32_t xcd_group(uint32_t b, uint32_t nblk, uint32_t run = kXcdGroup) {
-  const uint32_t g = 8u * run, sg = b / g;
+__device__ __forceinline__ uint32_t xcd_group(uint32_t b, uint32_t nblk) {
+  constexpr uint32_t g = 8u * kXcdGroup;
+  const uint32_t sg = b / g;
   if ((sg + 1) * g > nblk) return b;
   const uint32_t r = b - sg * g;
-  return sg * g + (r & 7u) * run + (r >> 3);
+  return sg * g + (r & 7u) * kXcdGroup + (r >> 3);
 }
 
 // The workgroup order of a cell launch, chosen by the host per launch (a.order):
