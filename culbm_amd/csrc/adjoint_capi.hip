@@ -392,7 +392,9 @@ int adjoint_impl(culbm_ctx* ctx, const culbm_adjoint_spec& sp, const double* wei
     launch_fused<S>(ctx, s);
     ++launches;
   };
-  const bool pairs = ctx->fused.pays && fused_scale_ok(ctx);
+  // (a mixed context with a depth takes pairs whatever the size, as its steps do)
+  const bool asked = c.opt_policy == CULBM_OPT_MIXED && c.wave_depth > 0;
+  const bool pairs = (ctx->fused.pays || asked) && fused_scale_ok(ctx);
   auto in_window = [&](int32_t t) { return t >= sp.t_begin && t <= sp.t_end; };
   // the first sweep accumulates J; the reverse sweep adds the objective's gradient to mu
   auto objective = [&](const void* f, float* m) {

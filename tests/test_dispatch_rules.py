@@ -87,3 +87,17 @@ def test_the_exported_schedule_is_the_one_that_runs():
                     assert lat.info()["launches_per_pass"] == len(want), what
                     lat.close()
     """)
+
+
+def test_adjoint_takes_pairs_where_the_context_asks_for_them():
+    fakehip.run("""
+    dim = (33, 21, 19)
+    for kw, pairs in [(dict(), 0), (dict(opt_policy=2), 0), (dict(opt_policy=2, wave_depth=6), 1),
+                      (dict(opt_policy=2, wave_depth=6, storage="fp16", storage_scale=0.5), 0)]:
+        for every in (0, 4):
+            lat = Lattice(LatticeConfig(domain=dim, **kw))
+            fake.fake_clear()
+            lat.adjoint(np.ones(lat.shape), 20, (20, 20), checkpoint_every=every, max_slots=0 if every else 3)
+            assert ("k_fused2" in launched()) == bool(pairs), (kw, every)
+            lat.close()
+    """)
