@@ -71,12 +71,20 @@ def test_pairs_equal_single_steps(dim, depth, storage, rounding):
     b.close()
 
 
+# Domains, and for each storage format from which one on (in this order) the
+# library takes pairs on 256 CUs.
+AUTO = [(61, 60, 59), (98, 97, 96), (203, 61, 90), (192, 160, 96), (192, 160, 144)]
+FIRST_IN_PAIRS = {("fp32", "nearest"): 1, ("fp16", "nearest"): 3, ("bf16", "nearest"): 3, ("fp16", "stochastic"): 4,
+                  ("bf16", "stochastic"): 4}
+
+
 @pytest.mark.parametrize("storage,rounding", STORAGE)
-@pytest.mark.parametrize("dim", [(98, 97, 96), (203, 61, 90), (192, 160, 96)])
+@pytest.mark.parametrize("dim", AUTO)
 def test_every_pull_policy_left_to_itself(dim, storage, rounding):
-    """Sizes around which the library starts to take pull steps in pairs: one
-    call of several steps, a pending dump and an odd step among them."""
+    """Sizes on both sides of where the library starts to take pull steps in pairs:
+    one call of several steps, a pending dump and an odd step among them."""
     st = state(*dim)
+    pairs = AUTO.index(dim) >= FIRST_IN_PAIRS[storage, rounding]
     a = make(st, storage=storage, rounding=rounding)
     a.step(1)
     a.dump()
@@ -86,12 +94,15 @@ def test_every_pull_policy_left_to_itself(dim, storage, rounding):
     a.close()
     for op in (0, 1, 2, 3):
         b = make(st, storage=storage, rounding=rounding, opt_policy=op)
+        if op:
+            assert (b.info()["launches_per_pass"] == 3) == pairs, op
         b.step(1)
         b.dump_deferred()
         b.step(6)
         assert np.array_equal(want, bits(b.get_ddf())), op
         for x, y in zip(b.macros(), fields):
             assert np.array_equal(bits(x), bits(y)), op
+        assert (b.profile_steps(2)["launches"] == 1) == pairs, op
         b.close()
 
 

@@ -316,10 +316,11 @@ def test_16bit_scale_is_derived_per_run():
 
 # ---- the optimised workload at full size --------------------------------------
 
+# (stream policy, opt policy, wavefront depth; 0: automatic)
 FULL_SIZE_FORMS = {
-    "fp32": [(1, 3), (0, 3), (0, 2), (1, 1), (1, 0)],
-    "fp16": [(1, 3), (0, 3), (0, 2)],
-    "bf16": [(1, 3)],
+    "fp32": [(0, 0, 0), (1, 3, 0), (0, 3, 0), (0, 2, 0), (1, 1, 0), (1, 0, 0), (0, 3, 16), (0, 1, 280)],
+    "fp16": [(0, 0, 0), (1, 3, 0), (0, 3, 0), (0, 2, 0), (0, 3, 16)],
+    "bf16": [(0, 0, 0), (1, 3, 0), (0, 1, 16)],
 }
 
 
@@ -328,7 +329,9 @@ FULL_SIZE_FORMS = {
                                                     ("fp16", "stochastic", 200), ("bf16", "nearest", 200)])
 def test_full_size_blocked_equals_plain(storage, rounding, steps):
     """288x272x280, 60 spheres, I = 5, automatic depths and workgroup orders (the
-    benchmark's configurations): every blocked and in-place form vs plain pull.
+    benchmark's configurations, and given depths, without which the pull policies
+    take pairs of steps here): every form vs plain pull steps asked for one at a
+    time, which the one-step kernel runs.
     The populations start at feq(rho, u) with rho = 1 + U(-1e-3, 1e-3) from a
     seed, so every cell, sphere and chunk seam carries non-zero, distinct values
     from the first step; FP32 runs the workload's 1000 steps."""
@@ -336,23 +339,27 @@ def test_full_size_blocked_equals_plain(storage, rounding, steps):
     rng = np.random.default_rng(21)
     st.rho[...] = (1.0 + rng.uniform(-1e-3, 1e-3, st.shape)).astype(np.float32)
 
-    def run(sp, op):
+    def run(sp, op, depth=0, singly=False):
         lat = make(st, init="feq", inv_tau=0.5, stream_policy=sp, opt_policy=op, inner_loop=5, storage=storage,
-                   rounding=rounding)
-        lat.step(steps)
+                   rounding=rounding, wave_depth=depth)
+        if sp == 0 and depth == 0:
+            assert lat.profile_steps(2)["launches"] == 1  # the pair kernel is the automatic route here
+            lat.init_ddf("feq")
+        for n in [1] * steps if singly else [steps]:
+            lat.step(n)
         lat.dump()
         r = (lat.macros(), lat.get_ddf())
         lat.close()
         return r
 
-    want_m, want_f = run(0, 0)
+    want_m, want_f = run(0, 0, singly=True)
     # the flow is developed everywhere: hardly a fluid cell has u_x exactly 0
     # (16-bit storage can cancel to an exact zero in a few cells of 20M)
     fluid = (st.flag & cases.DUMP) != 0
     assert np.count_nonzero(want_m[1][fluid] == 0.0) <= 1e-5 * np.count_nonzero(fluid)
-    for sp, op in FULL_SIZE_FORMS[storage]:
-        got_m, got_f = run(sp, op)
-        what = f"full-size ({sp},{op}) {storage} {rounding} {steps} steps"
+    for sp, op, depth in FULL_SIZE_FORMS[storage]:
+        got_m, got_f = run(sp, op, depth)
+        what = f"full-size ({sp},{op}) D={depth} {storage} {rounding} {steps} steps"
         for a, b in zip(got_m, want_m):
             assert_bitexact(a, b, what + " macros")
         assert_bitexact(got_f, want_f, what + " populations")
@@ -385,30 +392,33 @@ def test_precision_workload_512_blocked_equals_plain(storage):
 def test_mixed_with_inactive_cells_and_midrun_flag_change():
     """Cells without STORE keep their populations in both buffers; the fused
     two-step kernel reads them from src, plain pull alternates buffers: both
-    must agree, also after the flag field changes between runs."""
+    must agree, also after the flag field changes between runs.  A given depth makes
+    the steps run in pairs; without one they do not pay at this size."""
     st = obstacle_case(nx=70, ny=20, nz=17)
     rng = np.random.default_rng(9)
     st.flag[rng.random(st.shape) < 0.03] = 0
     flag2 = st.flag.copy()
     flag2[(rng.random(st.shape) < 0.02) & (flag2 != 0)] = cases.LOAD | cases.COLLIDE  # no STORE
     res = []
-    for op in (0, 2):
-        lat = make(st, init="feq", inv_tau=0.8, opt_policy=op, inner_loop=4)
+    for op, depth in ((0, 0), (2, 6), (2, 0)):
+        lat = make(st, init="feq", inv_tau=0.8, opt_policy=op, inner_loop=4, wave_depth=depth)
+        assert lat.info()["launches_per_pass"] == (2 if depth else 4 if op else 1)
         lat.step(6)
         lat.set_state(flag2, st.rho, st.vx, st.vy, st.vz)
         lat.step(7)
         lat.dump()
         res.append((lat.get_ddf(), lat.macros()))
         lat.close()
-    assert_bitexact(res[0][0], res[1][0], "populations")
-    for a, b in zip(res[0][1], res[1][1]):
-        assert_bitexact(a, b, "macros")
+    for ddf, macros in res[1:]:
+        assert_bitexact(res[0][0], ddf, "populations")
+        for a, b in zip(res[0][1], macros):
+            assert_bitexact(a, b, "macros")
 
 
 @pytest.mark.parametrize("storage,rounding", [("fp32", "nearest"), ("fp16", "stochastic")])
 def test_mixed_pairs_do_not_depend_on_call_boundaries(storage, rounding):
-    """The mixed policy takes its steps in pairs across passes and calls (one
-    plain step for an odd count): any split of 19 steps into calls, windows
+    """The mixed policy (here with a depth, which makes it) takes its steps in pairs
+    across passes and calls (one plain step for an odd count): any split of 19 steps into calls, windows
     included, gives the bits of 19 plain pull steps."""
     st = obstacle_case(nx=45, ny=26, nz=23)
     ref = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding)
@@ -416,14 +426,16 @@ def test_mixed_pairs_do_not_depend_on_call_boundaries(storage, rounding):
     want = ref.get_ddf()
     ref.close()
     for split in ([19], [1, 18], [5, 3, 9, 2], [2, 2, 2, 13], [7, 7, 5]):
-        lat = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding, opt_policy=2, inner_loop=5)
+        lat = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding, opt_policy=2, inner_loop=5,
+                   wave_depth=6)
         for n in split:
             lat.step(n)
-        assert lat.info()["step"] == 19
+        assert lat.info()["step"] == 19 and lat.info()["launches_per_pass"] == 3
         assert_bitexact(lat.get_ddf(), want, f"{storage} {rounding} split {split}")
         lat.close()
     # windows advance by innerLoop: three windows of 7 steps run 10 each
-    lat = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding, opt_policy=2, inner_loop=5)
+    lat = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding, opt_policy=2, inner_loop=5,
+               wave_depth=6)
     done = [lat.run_window(7)[0] for _ in range(3)]
     assert done == [10, 10, 10]
     ref = make(st, init="feq", inv_tau=0.7, storage=storage, rounding=rounding)
@@ -456,7 +468,8 @@ def test_ragged_domains_all_policies_match_the_oracle(dom):
     o.step(steps)
     want = o.ddf()
     for sp, op, il, wd in [(0, 0, 5, 0), (1, 0, 5, 0), (0, 3, 3, 0), (1, 3, 3, 1), (1, 3, 5, 0),
-                           (0, 1, 2, 0), (1, 1, 3, 2), (0, 2, 3, 0), (0, 2, 2, 1)]:
+                           (0, 1, 2, 0), (1, 1, 3, 2), (0, 2, 3, 0), (0, 2, 2, 1), (0, 2, 3, 2),
+                           (0, 3, 3, 1)]:
         lat = Lattice(LatticeConfig(domain=dom, inv_tau=0.8, stream_policy=sp, opt_policy=op,
                                     inner_loop=il, wave_depth=wd))
         lat.set_state(flag, rho, *u)
@@ -514,7 +527,7 @@ def test_16bit_ragged_domains_match_the_oracle(dom):
     steps = 7
     want = None
     for sp, op, il, wd in [(0, 0, 5, 0), (1, 0, 5, 0), (0, 3, 3, 0), (1, 3, 3, 1), (1, 3, 5, 0),
-                           (0, 1, 2, 0), (1, 1, 3, 2), (0, 2, 3, 0)]:
+                           (0, 1, 2, 0), (1, 1, 3, 2), (0, 2, 3, 0), (0, 2, 2, 1), (0, 2, 3, 2), (0, 3, 3, 1)]:
         lat = Lattice(LatticeConfig(domain=dom, inv_tau=0.8, stream_policy=sp, opt_policy=op,
                                     inner_loop=il, wave_depth=wd, storage="fp16"))
         lat.set_state(flag, rho, *u)
