@@ -12,7 +12,7 @@ Prints ONE JSON line: MLUPS of the headline form (value: the median of five
 device-timed 20-step windows after a warm-up window, in the developed flow:
 1000 untimed steps from rest come first), the HBM roofline of its
 dominant kernel (216 algorithmic bytes per FP32 cell-update, 108 for 16-bit
-storage), the other forms measured in the same run, the FP16 form's speed
+storage, half of that where a launch takes two steps), the other forms measured in the same run, the FP16 form's speed
 ratio and its error against the FP64 oracle, and the FP32 OpenMP CPU
 restatement timed on a bounded sample of the same workload.
 """
@@ -35,23 +35,24 @@ DOMAIN = (288, 272, 280)
 INV_TAU = 0.5
 
 FORMS = {
-    # name: (stream_policy, opt_policy, storage, description)
+    # name: (stream_policy, opt_policy, storage, description).  No depth is given, so
+    # every pull form leaves it to the library whether steps run in pairs.
     "fp32_inplace_blocked": (1, 3, "fp32", "FP32 in-place + dynamic (wavefront) temporal blocking"),
-    "fp32_plain_pull": (0, 0, "fp32", "FP32 plain pull, double buffer"),
+    "fp32_plain_pull": (0, 0, "fp32", "FP32 pull, double buffer, no blocking policy"),
     "fp32_inplace": (1, 0, "fp32", "FP32 in-place (esoteric twist), no blocking"),
     "fp32_inplace_static": (1, 1, "fp32", "FP32 in-place + static (cooperative) blocking"),
     "fp16_inplace_blocked": (1, 3, "fp16", "FP16-shifted in-place + dynamic blocking"),
     "bf16_inplace_blocked": (1, 3, "bf16", "BF16-shifted in-place + dynamic blocking"),
-    "fp16_plain_pull": (0, 0, "fp16", "FP16-shifted plain pull"),
-    "fp32_pull_blocked": (0, 3, "fp32", "FP32 pull + dynamic (wavefront) temporal blocking"),
-    "fp16_pull_blocked": (0, 3, "fp16", "FP16-shifted pull + dynamic blocking"),
-    "fp32_mixed": (0, 2, "fp32", "FP32 pull + mixed blocking (two steps per launch, LDS)"),
-    "fp16_mixed": (0, 2, "fp16", "FP16-shifted pull + mixed blocking (two steps per launch, LDS)"),
+    "fp16_plain_pull": (0, 0, "fp16", "FP16-shifted pull, no blocking policy"),
+    "fp32_pull_blocked": (0, 3, "fp32", "FP32 pull + dynamic policy"),
+    "fp16_pull_blocked": (0, 3, "fp16", "FP16-shifted pull + dynamic policy"),
+    "fp32_mixed": (0, 2, "fp32", "FP32 pull + mixed blocking (pairs of steps, LDS)"),
+    "fp16_mixed": (0, 2, "fp16", "FP16-shifted pull + mixed blocking (pairs of steps, LDS)"),
     "fp16_sr_inplace_blocked": (1, 3, "fp16", "FP16-shifted in-place + dynamic blocking, stochastic rounding",
                                 "stochastic"),
     "fp16_sr_mixed": (0, 2, "fp16", "FP16-shifted pull + mixed blocking, stochastic rounding", "stochastic"),
-    "fp16_sr_plain_pull": (0, 0, "fp16", "FP16-shifted plain pull, stochastic rounding", "stochastic"),
-    "bf16_mixed": (0, 2, "bf16", "BF16-shifted pull + mixed blocking (two steps per launch, LDS)"),
+    "fp16_sr_plain_pull": (0, 0, "fp16", "FP16-shifted pull, no blocking policy, stochastic rounding", "stochastic"),
+    "bf16_mixed": (0, 2, "bf16", "BF16-shifted pull + mixed blocking (pairs of steps, LDS)"),
 }
 HEADLINE = "fp32_inplace_blocked"
 
@@ -106,8 +107,10 @@ def run_form(state, name, steps, warmup, inner_loop, windows=5, window_steps=20,
     lat.close()
     med = sorted(win)[len(win) // 2]  # the median window (odd count)
     mlups, win_ms, win_steps = med
-    bpu = 27 * 2 * info["bytes_per_pop"]  # algorithmic bytes per cell-update
     launches_per_step = prof["launches"] / prof["steps"]
+    pairs = prof["launches"] < prof["steps"]  # a launch takes two steps (k_fused2)
+    # algorithmic bytes per cell-update: a launch reads and writes every population once
+    bpu = 27 * 2 * info["bytes_per_pop"] // (2 if pairs else 1)
     return {
         "mlups": mlups,
         "window_mlups": [round(w[0], 1) for w in win],
@@ -118,12 +121,13 @@ def run_form(state, name, steps, warmup, inner_loop, windows=5, window_steps=20,
         "bytes_per_update": bpu,
         "effective_gbs": mlups * 1e6 * bpu / 1e9,
         # average launch of the median window (its event pair over its launch
-        # count: one kernel per form except mixed, whose windows also hold the
-        # odd pull steps) and the per-launch event figure (adds ~2.7 us per launch)
+        # count: one kernel per form, but an odd step of a form that runs in pairs
+        # runs alone) and the per-launch event figure (adds ~2.7 us per launch)
         "window_launch_avg_us": win_ms * 1e3 / (launches_per_step * win_steps),
         "kernel_gbs": bpu * ncell * prof["steps"] / (prof["kernel_ms"] * 1e-3) / 1e9,
         "kernel_avg_us": prof["kernel_ms"] * 1e3 / prof["launches"],
         "launches_per_step": launches_per_step,
+        "pairs": pairs,
         "wave_depth": info["wave_depth"],
         "frac_hbm": mlups * 1e6 * bpu / 1e9 / HBM_PEAK_GBS,
     }
@@ -428,9 +432,9 @@ def main(argv=None) -> int:
                                          and e["u_max_over_u_in"] <= 1e-3)
 
     # dominant kernel's rate: algorithmic bytes per launch over the average launch
-    # duration of the median window (its event pair over its launch count; the
-    # mixed form's windows also hold k_pull, so it takes per-launch events)
-    single = FORMS[ns.form][1] != 2
+    # duration of the median window (its event pair over its launch count; a form
+    # that runs in pairs takes per-launch events, an odd step of its windows is k_pull)
+    single = not head["pairs"]
     achieved = head["effective_gbs"] if single else head["kernel_gbs"]
     avg_us = head["window_launch_avg_us"] if single else head["kernel_avg_us"]
     # HBM bytes per launch of the dominant kernel: the counter-derived bytes per

@@ -49,3 +49,21 @@ def test_fp16_claim_forms_are_stochastic_fp16():
     for form in bench.FP16_CLAIMS:
         spec = bench.FORMS[form]
         assert spec[2] == "fp16" and len(spec) > 4 and spec[4] == "stochastic", form
+
+
+def test_algorithmic_bytes_follow_the_steps_of_a_launch():
+    """A launch of two steps moves half the bytes per update, whichever policy it
+    runs under, so no form's share of the peak can pass 1 by its bookkeeping."""
+    import fakehip
+
+    fakehip.run("""
+    sys.modules["torch"] = None  # bench synchronises through it where it is there
+    import bench
+    for dim, pull_in_pairs in (((112, 104, 96), True), ((40, 40, 40), False)):
+        st = cases.channel(*dim)
+        for name in ("fp32_plain_pull", "fp32_pull_blocked", "fp32_mixed", "fp32_inplace_blocked", "fp32_inplace"):
+            r = bench.run_form(st, name, 10, 2, 5, develop=4)
+            pairs = pull_in_pairs and "inplace" not in name
+            assert r["pairs"] == pairs and r["bytes_per_update"] == (108 if pairs else 216), (dim, name, r)
+            assert (r["launches_per_step"] == 0.5) == pairs
+    """)
