@@ -17,8 +17,8 @@
 // Layout: every buffer here uses the dense pull layout (px = nx, py = ny,
 // direction stride = cells); populations in the storage format S, mu in FP32.
 // Gradients accumulate in FP64: one accumulator per EQU cell and input, one per
-// workgroup for invTau and J, each summed in a fixed order, so a run is
-// bit-reproducible.
+// 256-cell block for invTau, one per 64 weighted cells for J, each summed in a
+// fixed order, so a run is bit-reproducible.
 // Included by capi.hip after lbm_kernels.hip.
 
 namespace culbm {
@@ -32,7 +32,7 @@ struct AdjArgs {
   int64_t n_equ;
   float* carry;          // [27][n_keep] running lambda of the cells without STORE, or null
   int64_t n_keep;
-  double* tau_acc;       // one accumulator per workgroup
+  double* tau_acc;       // one accumulator per block of cells
   const float* wobj;     // objective weights (FP32, per cell) when t is in the window, else null
 };
 
