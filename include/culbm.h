@@ -253,7 +253,7 @@ typedef struct culbm_adjoint_stats {
  * outside EQU cells.  grad_f0: 27*nx*ny*nz floats ([27][nz][ny][nx]) or NULL;
  * required when spec->want_f0.  Fails with CULBM_ERR_INVALID when the
  * checkpoints do not fit mem_cap.  A workspace of up to 1 GiB stays with the
- * context for its next call, 1 GiB in all on a device; it is freed by
+ * context for its next call, 8 GiB in all on a device; it is freed by
  * culbm_destroy, when other contexts' take its place, and where an allocation of
  * the library would fail. */
 int culbm_adjoint(culbm_ctx* ctx, const culbm_adjoint_spec* spec, const double* weight,

@@ -44,12 +44,14 @@ def test_kept_workspaces_are_bounded_per_device_and_given_back():
         lat.adjoint(np.ones(lat.shape), steps, (1, steps), checkpoint_every=1)
         return lat
 
-    lats = [made((64, 60, 50), 18) for _ in range(4)]  # about 0.44 GB of workspace each
+    lats = [made((64, 60, 50), 18) for _ in range(21)]  # about 0.44 GB of workspace each
     own = [lat.info()["device_bytes"] for lat in lats]
     assert sum(own) == fake.fake_bytes()
     base = min(own)
     kept = [b - base for b in own]
-    assert kept[:2] == [0, 0] and min(kept[2:]) > 0.4e9 and sum(kept) <= GiB, kept
+    first = sum(k == 0 for k in kept)
+    assert 0 < first and kept[:first] == [0] * first and min(kept[first:]) > 0.4e9, kept
+    assert 7.5 * GiB < sum(kept) <= 8 * GiB, kept
     # an allocation that only fits once they are given back, by a context that keeps
     # none, by one that does and by a new one
     plain = 27 * 4 * 64 * 60 * 50
@@ -57,11 +59,11 @@ def test_kept_workspaces_are_bounded_per_device_and_given_back():
                  lambda: lats[0].init_ddf("feq"), lats[0].moment_sums,
                  lambda: Lattice(LatticeConfig(domain=(16, 16, 16))).close()):
         fake.fake_limit(1 << 40)
-        lats[3].adjoint(np.ones(lats[3].shape), 18, (1, 18), checkpoint_every=1)
-        assert lats[3].info()["device_bytes"] > base
+        lats[-1].adjoint(np.ones(lats[-1].shape), 18, (1, 18), checkpoint_every=1)
+        assert lats[-1].info()["device_bytes"] > base
         fake.fake_limit(fake.fake_bytes())
         call()
-        assert lats[3].info()["device_bytes"] == base
+        assert lats[-1].info()["device_bytes"] == base
     # one that never fits still fails, and the context goes on
     fake.fake_limit(fake.fake_bytes() + plain // 2)
     try:
