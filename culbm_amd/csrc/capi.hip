@@ -1038,11 +1038,12 @@ int alloc(culbm_ctx* ctx, void** p, size_t bytes) {
 }
 
 // Bytes of populations (as allocated) and flags up to which the Infinity Cache
-// (256 MB) serves one step what the step before it wrote: the middle of a range in
-// which sizes run two ways.  In place see auto_depth; plain pull steps run 49k to
-// 55k MLUPS in 16 bits up to 200 MB, 44k to 55k from there to 250 MB and 43k to 45k
-// at 257 MB, in FP32 29k at 224 MB, 25k to 28k at 237 to 253 MB, 23k at 283 MB.
-constexpr double kCacheHolds = 237e6;
+// (256 MB) serves one step what the step before it wrote, wherever the buffers lie.
+// From there to about 240 MB it depends on where they lie (in place see auto_depth;
+// plain pull steps run 49k to 55k MLUPS in 16 bits up to 200 MB, 44k to 55k from
+// there to 250 MB and 43k to 45k at 257 MB, in FP32 29k at 224 MB, 25k to 28k at 237
+// to 253 MB, 23k at 283 MB).
+constexpr double kCacheHolds = 227e6;
 
 // Planes per wavefront chunk.  FP32 in place and pull: a launch-size target
 // (1.4M cells in place, 1.25M pull) capped by the cache-fitting depth (D + T + 1
@@ -1067,11 +1068,12 @@ int32_t auto_depth(const culbm_ctx* ctx) {
     return std::max(2, std::min(d, nz));
   }
   // FP32 in place: a domain that the cache holds is one launch a step.  Against the
-  // chunk rule's two launches, 8 contexts a size: 31 sizes from 125 to 236 MB +2 to
-  // +10 % (128^3, 234 MB, 28.1k vs 27.5k MLUPS; 157x93x141, 233 MB, 25.4k vs
-  // 24.4k; 200x104x100, 232 MB, 28.7k vs 27.6k) but 136x128x120 and 123x127x130
-  // -1 to +3 % and 101x140x133 -5 to -12 %; of 13 sizes from 237 to 266 MB, 10
-  // -6 to -18 % (128x128x132, 241 MB, 23.7k vs 26.5k), 3 below 240 MB +2 to +4 %.
+  // chunk rule's two launches, 8 contexts a size, on one to four boxes: 22 sizes from
+  // 125 to 226 MB +1 to +10 % (128x128x120, 219 MB, 29.1k vs 28.0k MLUPS; 144x118x118,
+  // 224 MB, 28.4k vs 27.8k) but 96x150x140 -2 to +2 %.  From 230 to 237 MB a process
+  // runs fast or slow by where its buffers lie, 0 % on average: 128^3, 234 MB, 28.8k or
+  // 23.1k vs 27.5k, 157x93x141, 233 MB, 25.4k or 23.6k vs 24.4k, 136x128x120 27.4k or
+  // 23.1k vs 26.8k.  Of 13 sizes from 237 to 266 MB 10 lost 6 to 18 %.
   if (ctx->inplace && 27.0 * ctx->bpp * double(ctx->dstride) + cells * nz <= kCacheHolds) return nz;
   const double plane = cells * (27.0 * ctx->bpp * (ctx->inplace ? 1 : 2) + 1.0);
   const double budget = 160.0 * 1024 * 1024;
@@ -1166,7 +1168,7 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
     }
   }
   const double held = (2.0 * 27.0 * ctx->bpp + 1.0) * cells / kCacheHolds;
-  const double past = std::min(std::max((held - 0.84) / 0.32, 0.0), 1.0);
+  const double past = std::min(std::max((held - 0.88) / 0.33, 0.0), 1.0);
   const double cell_us = 1e-6 * (wide ? 30.0 + 12.0 * past : 18.0 + 3.6 * past);
   // Non-temporal stores leave the L2 to the halo lines and miss the cache: FP32
   // rows of whole 64-byte blocks gain once the cache holds little of the two
@@ -1175,7 +1177,7 @@ FusedPlan fused_plan(const culbm_ctx* ctx, int ncu) {
   // 192x160x176 38.9k, 39.7k; 256^3 37.6k, 40.3k; 288x272x280 42.6k, 43.2k);
   // blocks shared by two tiles are then written twice (203x170x119 34.9k, 25.3k),
   // and 16-bit rows go either way.
-  best.nt = wide && held > 1.3 && c.nx % 16 == 0 && best.tx % 16 == 0;
+  best.nt = wide && held > 1.36 && c.nx % 16 == 0 && best.tx % 16 == 0;
   const double far_line = c.storage == CULBM_STORAGE_BF16 ? 0.92 : 0.95;
   const double line = ctx->sr ? 1.0 : 1.09 + (far_line - 1.09) * past;
   // a launch's own start and fill count where it is short

@@ -6,7 +6,7 @@ import fakehip
 
 
 def test_in_place_one_launch_a_step_follows_the_allocated_bytes():
-    """FP32 in place, no depth given, domains of 1.7M to 2.4M cells around the
+    """FP32 in place, no depth given, domains of 1.6M to 2.4M cells around the
     line, odd widths (padded rows) and even ones (packed) among them."""
     fakehip.run("""
     import random
@@ -14,14 +14,14 @@ def test_in_place_one_launch_a_step_follows_the_allocated_bytes():
     dims = [(101, 140, 141), (128, 128, 128), (157, 93, 141), (140, 120, 126), (128, 128, 132), (96, 150, 148)]
     while len(dims) < 24:
         nx, ny = rng.randrange(60, 220), rng.randrange(60, 220)
-        nz = round(rng.uniform(215e6, 255e6) / 109 / (nx + 1) / (ny + 1))
+        nz = round(rng.uniform(185e6, 240e6) / 109 / (nx + 1) / (ny + 1))
         if nz > 40:
             dims.append((nx, ny, nz))
     one = 0
     for nx, ny, nz in dims:
         lat = Lattice(LatticeConfig(domain=(nx, ny, nz), stream_policy=1, opt_policy=3, inner_loop=5))
         populations = lat.info()["device_bytes"] - nx * ny * nz * 20 - (nx * ny * nz + 3) // 4 * 4
-        whole = populations + nx * ny * nz <= 237e6
+        whole = populations + nx * ny * nz <= 227e6
         one += whole
         assert (lat.info()["launches_per_pass"] == 5) == whole, (nx, ny, nz, populations)
         lat.close()
