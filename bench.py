@@ -108,7 +108,10 @@ def run_form(state, name, steps, warmup, inner_loop, windows=5, window_steps=20,
     med = sorted(win)[len(win) // 2]  # the median window (odd count)
     mlups, win_ms, win_steps = med
     launches_per_step = prof["launches"] / prof["steps"]
-    pairs = prof["launches"] < prof["steps"]  # a launch takes two steps (k_fused2)
+    # does a launch take two steps (k_fused2)?  The static policy's replayed graph is
+    # one event pair a pass; the library's own count of its launches tells it apart
+    graph = op == 1 and inner_loop > 1 and info["launches_per_pass"] >= inner_loop
+    pairs = not graph and prof["launches"] == (prof["steps"] + 1) // 2 and prof["steps"] > 1
     # algorithmic bytes per cell-update: a launch reads and writes every population once
     bpu = 27 * 2 * info["bytes_per_pop"] // (2 if pairs else 1)
     return {

@@ -61,9 +61,10 @@ def test_algorithmic_bytes_follow_the_steps_of_a_launch():
     import bench
     for dim, pull_in_pairs in (((112, 104, 96), True), ((40, 40, 40), False)):
         st = cases.channel(*dim)
-        for name in ("fp32_plain_pull", "fp32_pull_blocked", "fp32_mixed", "fp32_inplace_blocked", "fp32_inplace"):
+        for name in ("fp32_plain_pull", "fp32_pull_blocked", "fp32_mixed", "fp32_inplace_blocked", "fp32_inplace",
+                     "fp32_inplace_static"):
             r = bench.run_form(st, name, 10, 2, 5, develop=4)
             pairs = pull_in_pairs and "inplace" not in name
             assert r["pairs"] == pairs and r["bytes_per_update"] == (108 if pairs else 216), (dim, name, r)
-            assert (r["launches_per_step"] == 0.5) == pairs
+            assert (r["launches_per_step"] == 0.5) == pairs, (dim, name, r)
     """)
