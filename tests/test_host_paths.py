@@ -1,5 +1,6 @@
 """Host side of the C ABI on the stand-in runtime (no GPU, kernels do not run):
-device memory held and given back."""
+device memory held and given back, host allocations that fail, the routes and
+threads of copies to the host."""
 from __future__ import annotations
 
 import fakehip
