@@ -948,8 +948,8 @@ size_t ddf_bytes(const culbm_ctx* ctx) { return size_t(27) * size_t(ctx->dstride
 // so any thread may free it: a context that keeps one (of up to kAdjKeep bytes)
 // makes room by freeing the others' oldest beyond kAdjKeepAll bytes on the device,
 // 3 % of its memory, and an allocation that fails frees them all and is made again.
-// (With 1 GiB in all, contexts used in turn took each other's: 104x51x116 FP16,
-// 540 MB a context, 17.5 -> 19.6 ms a gradient.)
+// (With 1 GiB in all, three contexts used in turn took each other's: 118x110x29
+// FP16, 650 MB a context, 10.4 ms a gradient, 10.0 with 8 GiB.)
 constexpr int64_t kAdjKeep = int64_t(1) << 30, kAdjKeepAll = int64_t(8) << 30;
 std::mutex g_kept_mu;
 culbm_ctx* g_kept = nullptr;  // oldest first
@@ -1068,7 +1068,7 @@ int32_t auto_depth(const culbm_ctx* ctx) {
     return std::max(2, std::min(d, nz));
   }
   // FP32 in place: a domain that the cache holds is one launch a step.  Against the
-  // chunk rule's two launches, 8 contexts a size, on one to four boxes: 22 sizes from
+  // chunk rule's two launches, 8 contexts a size, on one to four cards: 22 sizes from
   // 125 to 226 MB +1 to +10 % (128x128x120, 219 MB, 29.1k vs 28.0k MLUPS; 144x118x118,
   // 224 MB, 28.4k vs 27.8k) but 96x150x140 -2 to +2 %.  From 230 to 237 MB a process
   // runs fast or slow by where its buffers lie, 0 % on average: 128^3, 234 MB, 28.8k or
